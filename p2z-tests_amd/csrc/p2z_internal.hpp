@@ -24,8 +24,7 @@ struct LaunchCfg {
 
 // Hit-staging depth of the fused pass when none is set: FAST runs 5 waves per
 // SIMD at depth 1 (89 VGPRs) against 4 at depth 2 (100) and measures 1-3%
-// faster; the reference mode (92 / 100 VGPRs: 5 waves against 4) 1-3% faster
-// at depth 1 on three boxes; the FP64-gain mode (126 / 138 VGPRs: 4 waves
+// faster; the reference mode (100 / 112 VGPRs) runs at depth 1; the FP64-gain mode (126 / 138 VGPRs: 4 waves
 // against 3) within 1% either way, and keeps depth 2.
 inline int default_hit_stage(int math) { return math == 2 ? 2 : 1; }
 

@@ -64,6 +64,34 @@ __device__ inline Hit load_hit(const float* __restrict__ hb) {
   return h;
 }
 
+// Whether a track's layers have to be computed again in the reference
+// typing's full form (redo_ref); no other arithmetic marks tracks.
+template <int kMath>
+__device__ inline bool marked(const Track& t, const Carry<kMath>& g) {
+  if constexpr (kMath == kRef)
+    return g.redo || !ref_finite(t);
+  else
+    return false;
+}
+
+// The n layers of a marked track again, from its input state and in the full
+// form: the exception (an operand that overflows or is not finite).
+template <int W>
+__device__ inline void redo_ref(Track& t, const float* __restrict__ tb, const float* __restrict__ hb, int n) {
+  // the address hidden from common-subexpression elimination: otherwise the
+  // track's input would be kept in registers through all layers for this load
+  asm volatile("" : "+v"(tb));
+  load_track<W>(t, tb);
+  const RefCarry c = ref_carry(t);
+  Hit next{};
+  if (0 < n) next = load_hit<W>(hb);
+  for (int lay = 0; lay < n; ++lay) {
+    const Hit h = next;
+    if (lay + 1 < n) next = load_hit<W>(hb + (int64_t)(lay + 1) * (kHitWords * W));
+    step_ref_full(t, h, c);
+  }
+}
+
 // Layers [0, n) of one track whose hits start at hb (consecutive layers 9W
 // words apart), with the hits of the next kDepth layers (1 or 2) in flight
 // while a layer is computed.  The loop is unrolled by kDepth + 1 over
@@ -73,12 +101,12 @@ __device__ inline Hit load_hit(const float* __restrict__ hb) {
 // differ and each lane's loads and steps stop at its own n.  Every load index
 // is < n.
 template <int W, int kMath, int kDepth, bool kPerLane>
-__device__ __forceinline__ void run_layers(Track& t, const float* __restrict__ hb, int n, int nmax) {
+__device__ __forceinline__ bool run_layers(Track& t, const float* __restrict__ hb, int n, int nmax) {
   static_assert(kDepth == 1 || kDepth == 2, "prefetch depth 1 or 2");
-  if (nmax <= 0) return;
+  if (nmax <= 0) return false;
   auto at = [&](int lay) { return load_hit<W>(hb + (int64_t)lay * (kHitWords * W)); };
   auto live = [&](int lay) { return kPerLane ? lay < n : true; };
-  Trig g;
+  Carry<kMath> g;
   Hit a{}, b{};
   if (live(0)) a = at(0);
   if (1 < nmax && live(1)) b = at(1);
@@ -108,6 +136,7 @@ __device__ __forceinline__ void run_layers(Track& t, const float* __restrict__ h
     if (lay < nmax && live(lay)) layer_step<kMath, false>(t, b, g);
     if (lay + 1 < nmax && live(lay + 1)) layer_step<kMath, false>(t, c, g);
   }
+  return marked<kMath>(t, g);
 }
 
 // Ragged form of run_layers: lane layer counts n <= nmax differ, the loop
@@ -116,11 +145,11 @@ __device__ __forceinline__ void run_layers(Track& t, const float* __restrict__ h
 // next kDepth layers are in flight while a layer is computed; a single step
 // instance keeps the register count down where the steps are masked.
 template <int W, int kMath, int kDepth>
-__device__ __forceinline__ void run_layers_lanes(Track& t, const float* __restrict__ hb, int n, int nmax) {
+__device__ __forceinline__ bool run_layers_lanes(Track& t, const float* __restrict__ hb, int n, int nmax) {
   static_assert(kDepth == 1 || kDepth == 2, "prefetch depth 1 or 2");
-  if (nmax <= 0) return;
+  if (nmax <= 0) return false;
   auto at = [&](int lay) { return load_hit<W>(hb + (int64_t)lay * (kHitWords * W)); };
-  Trig g;
+  Carry<kMath> g;
   Hit h0{}, h1{}, h2{};
   if (0 < n) h0 = at(0);
   if (1 < n) h1 = at(1);
@@ -136,6 +165,7 @@ __device__ __forceinline__ void run_layers_lanes(Track& t, const float* __restri
     }
     if (lay < n) layer_step<kMath, false>(t, h0, g);
   }
+  return marked<kMath>(t, g);
 }
 
 // Maximum of v over the 64 lanes of the wave (every lane must be active).
@@ -158,8 +188,12 @@ __global__ __launch_bounds__(256) void k_fused(const float* __restrict__ trk,
   const int64_t b = g / W;
   const int l = (int)(g % W);
   Track t;
-  load_track<W>(t, trk + b * (kTrkWords * W) + l);
-  run_layers<W, kMath, kDepth, false>(t, hit + b * (int64_t)nlayer * (kHitWords * W) + l, nlayer, nlayer);
+  const float* tb = trk + b * (kTrkWords * W) + l;
+  const float* hb = hit + b * (int64_t)nlayer * (kHitWords * W) + l;
+  load_track<W>(t, tb);
+  const bool redo = run_layers<W, kMath, kDepth, false>(t, hb, nlayer, nlayer);
+  if constexpr (kMath == kRef)
+    if (redo) redo_ref<W>(t, tb, hb, nlayer);
   store_track<W>(t, out + b * (kTrkWords * W) + l);
 }
 
@@ -182,16 +216,20 @@ __device__ __forceinline__ void ragged_item(const float* __restrict__ trk, const
   Track t{};
   int n = 0;
   const float* hb = hit;
+  const float* tb = trk;
   BlockDesc d{};
   if (valid) {
     d = blocks[di];
-    load_track<W, true>(t, trk + d.trk_block * (kTrkWords * W) + l);
+    tb = trk + d.trk_block * (kTrkWords * W) + l;
+    load_track<W, true>(t, tb);
     n = lane_nlay[d.trk_block * W + l];
     n = n < d.nlayer ? n : d.nlayer;
     n = n > 0 ? n : 0;
     hb = hit + d.hit_block * (kHitWords * W) + l;
   }
-  run_layers_lanes<W, kMath, kPrefetch>(t, hb, n, wave_max(n));
+  const bool redo = run_layers_lanes<W, kMath, kPrefetch>(t, hb, n, wave_max(n));
+  if constexpr (kMath == kRef)
+    if (valid && redo) redo_ref<W>(t, tb, hb, n);
   if (valid) store_track<W>(t, out + d.out_block * (kTrkWords * W) + l);
 }
 
@@ -382,14 +420,18 @@ __device__ __forceinline__ void serve_item(const ServeLaunch& a, uint64_t k, int
   Track t{};
   int n = 0;
   const float* hb = a.hit;
+  const float* tin = a.trk;
   if (valid) {
-    load_track<W, true>(t, a.trk + tb * (kTrkWords * W) + l);
+    tin = a.trk + tb * (kTrkWords * W) + l;
+    load_track<W, true>(t, tin);
     n = a.lanes[tb * W + l];
     n = n < nl ? n : nl;
     n = n > 0 ? n : 0;
     hb = a.hit + hblk * (kHitWords * W) + l;
   }
-  run_layers_lanes<W, kMath, kPrefetch>(t, hb, n, wave_max(n));
+  const bool redo = run_layers_lanes<W, kMath, kPrefetch>(t, hb, n, wave_max(n));
+  if constexpr (kMath == kRef)
+    if (valid && redo) redo_ref<W>(t, tin, hb, n);
   if (valid) store_track_through<W>(t, a.out + ob * (kTrkWords * W) + l);
   wait_stores();
   if (lane == 0) {
@@ -493,9 +535,10 @@ __global__ __launch_bounds__(256) void k_propagate(const float* inErr, const flo
   for (int e = 0; e < 6; ++e) t.p[e] = inPar[o + e * W];
   t.q = inChg[o];
   const float hz = msP[b * hs + 2 * W + l];
-  if constexpr (kMath == kRef)
-    propagate_ref(t, hz);
-  else
+  if constexpr (kMath == kRef) {
+    bool unused = true;
+    propagate_ref<false>(t, hz, ref_carry(t), unused);
+  } else
     propagate_fast<false, kMath == kFp64Gain>(t, hz);
 #pragma unroll
   for (int e = 0; e < 21; ++e) outErr[o + e * W] = t.P[e];
@@ -526,9 +569,10 @@ __global__ __launch_bounds__(256) void k_update(float* trkErr, float* inPar, con
   h.xx = hitErr[ho];
   h.xy = hitErr[ho + W];
   h.yy = hitErr[ho + 2 * W];
-  if constexpr (kMath == kRef)
-    update_ref(t, h);
-  else if constexpr (kMath == kFast)
+  if constexpr (kMath == kRef) {
+    bool unused = true;
+    update_ref<false>(t, h, unused);
+  } else if constexpr (kMath == kFast)
     update_fast<false>(t, h);
   else
     update_fp64gain<false>(t, h);

@@ -12,7 +12,8 @@
 //               reference's summation order, and sin/cos with the bits of
 //               the C library the reference calls (glibc's sinf/cosf,
 //               p2z_libm.hpp).  It reproduces the reference build bit for
-//               bit.
+//               bit; layers after the first leave out the terms whose
+//               zeros cannot change a bit (propagate_ref).
 //   kFast     : FP32 with FMA contraction, native reciprocals and the sparse
 //               structure of the Jacobian and of the covariance exploited.
 //   kFp64Gain : kFast propagation; the 2x2 residual-covariance inverse, the
@@ -57,32 +58,128 @@ struct Hit {
 // kRef: reference typing
 // ---------------------------------------------------------------------------
 
-__device__ inline void propagate_ref(Track& t, float hz) {
+// 1/x to the nearest float: the hardware reciprocal (1 ulp) refined by one
+// Newton step with a fused multiply-add, for |x| in [2^-100, 2^100].  Equal to
+// (float)(1. / (double)x) on every float of that range (checked on the GPU
+// over all mantissas and exponents): 1/x of a 24-bit x is never closer than
+// 2^-49 to the middle of two floats, so the double division the reference
+// writes does not round twice.  The 1-ulp estimate alone is biased low and
+// would shift all tracks of an event, which share nearly the same ipt and
+// cos(theta), the same way.
+__device__ inline float fast_rcp(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(r, __builtin_fmaf(-x, r, 1.0f), r);
+}
+
+// The divisions of operands that real tracks never have, out of line: inline,
+// their registers would add to the layer loops' peak.
+__device__ __noinline__ float ref_rcp_any(float x) { return (float)(1. / (double)x); }
+__device__ __noinline__ float ref_inv_det_any(double det) { return (float)(1. / det); }
+
+// (float)(1. / (double)x), the reference's float reciprocals.
+__device__ inline float ref_rcp(float x) {
+  const float a = __builtin_fabsf(x);
+  if (__builtin_expect(!(a > 0x1p-100f && a < 0x1p100f), 0)) return ref_rcp_any(x);
+  return fast_rcp(x);
+}
+
+// (float)(1. / det) for |det| in (2^-120, 2^120): the hardware's FP64
+// reciprocal (error below 2^-24, measured) refined by two Newton steps, so
+// that its last rounding sees 1/det within 2^-86.  The float differs from the
+// correctly rounded quotient's only if 1/det lies that close to a boundary of
+// the rounding to double next to the middle of two floats; an enumeration of
+// the 2^25 such boundaries finds no double det whose reciprocal does.
+__device__ inline float ref_inv_det(double det) {
+  double y = __builtin_amdgcn_rcp(det);
+  y = __builtin_fma(__builtin_fma(-det, y, 1.0), y, y);
+  y = __builtin_fma(__builtin_fma(-det, y, 1.0), y, y);
+  return (float)y;
+}
+
+// Per-track constants of the reference typing and the mark of a track that
+// the short form of the layer step (kZ0, below) does not reproduce.
+//   rkd: 1/k in double.  (float)((double)a * rkd) is a / k rounded to nearest
+//   for a normal quotient: the product is within 2^-52 of a / k, and the
+//   quotient of two floats is never closer than 2^-49 to the middle of two.
+struct RefCarry {
+  float k = 0.f;
+  double rkd = 0.;
+  bool redo = false;
+};
+
+// kZ0, the layers of a track after its first: the z row and column of P are
+// +0 and no other entry is -0.  Every term with them is then a zero added to
+// a partial sum that is not -0, which leaves the sum's bits as they are, so it
+// is left out; what it leaves keeps both properties (a sum is -0 only if its
+// first term is, x - y only if x is).  That holds while the Jacobian is
+// finite and the products with the zeros are zeros: ok is cleared where
+// operands are outside ranges that bound every Jacobian entry below 2^127
+// (|ipt|, |1/ipt|, |1/cosT|, |dz| < 2^30) or z is a zero (the update adds a
+// zero of either sign to it); where the update meets a value that is not
+// finite, or an operand is NaN, a diagonal entry of P or a position ends up
+// not finite and stays so, which the caller sees at the end (ref_finite).
+// Such tracks are computed again with the full form.
+// Bound: VALU issue, 671 instructions per layer before, about 460 now, with the
+// branch-free sin/cos and the reciprocals above.  100 events x 9600 tracks x
+// 20 layers: 0.260-0.266 -> 0.202 ms; 7 x 5008 x 26 at W = 16: 41 -> 27 us.
+// Angles are not restricted: low-momentum tracks near theta = pi/2 wind phi up
+// by hundreds of radians and throw theta about.  Marking those with an angle
+// above 120 took 40 events of the wide-range workload from 139 us to 164; with
+// the library's large-argument path in the layer they take 124.
+template <bool kZ0>
+__device__ inline void propagate_ref(Track& t, float hz, const RefCarry& carry, bool& ok) {
 #pragma clang fp contract(off)
   float* p = t.p;
   float* P = t.P;
   const float zout = hz;
-  const float k = t.q * kKfact;
+  const float k = carry.k;
   const float deltaZ = zout - p[2];
   const float ipt = p[3];
-  const float pt = (float)(1. / (double)ipt);
   float sinP, cosP, sinT, cosT;
-  sincosf_glibc(p[4], &sinP, &cosP);
-  sincosf_glibc(p[5], &sinT, &cosT);
+  // sincosf_glibc of both angles with one branch for its rare range (a NaN
+  // comes out as NaN of either)
+  glibc_sincosf::sincosf_below_120(p[4], &sinP, &cosP);
+  glibc_sincosf::sincosf_below_120(p[5], &sinT, &cosT);
+  if (__builtin_expect(!(fmaxf(__builtin_fabsf(p[4]), __builtin_fabsf(p[5])) < 120.f), 0)) {
+    if (!(__builtin_fabsf(p[4]) < 120.f)) {
+      const glibc_sincosf::Poly v = glibc_sincosf::sincosf_large(p[4]);
+      sinP = v.s;
+      cosP = v.c;
+    }
+    if (!(__builtin_fabsf(p[5]) < 120.f)) {
+      const glibc_sincosf::Poly v = glibc_sincosf::sincosf_large(p[5]);
+      sinT = v.s;
+      cosT = v.c;
+    }
+  }
+  const float pt = kZ0 ? fast_rcp(ipt) : ref_rcp(ipt);
   const float pxin = cosP * pt;
   const float pyin = sinP * pt;
-  const float icosT = (float)(1.0 / (double)cosT);
-  const float icosTk = icosT / k;
+  const float icosT = kZ0 ? fast_rcp(cosT) : ref_rcp(cosT);
+  const float icosTk = (float)((double)icosT * carry.rkd);
   const float alpha = deltaZ * sinT * ipt * icosTk;
-  float sina, cosa;
-  sincosf_glibc(alpha, &sina, &cosa);
+  if constexpr (kZ0) {
+    ok &= __builtin_fabsf(deltaZ) < 0x1p30f;
+    ok &= __builtin_fabsf(ipt) < 0x1p30f;
+    ok &= __builtin_fabsf(pt) < 0x1p30f;
+    ok &= __builtin_fabsf(icosT) < 0x1p30f;
+    ok &= zout != 0.f;
+  }
+  // The turning angle of one layer and cosP sina: below 0.75 in every lane of
+  // the wave (then |cosP sina| < 0.69), as layers a few ten cm apart have it,
+  // neither needs a reduction.
+  float sina, cosa, sC, cC;
+  if (__builtin_amdgcn_ballot_w64(!(__builtin_fabsf(alpha) < 0.75f)) == 0) {
+    glibc_sincosf::sincosf_small(alpha, &sina, &cosa);
+    glibc_sincosf::sincosf_small(cosP * sina, &sC, &cC);
+  } else {
+    sincosf_glibc(alpha, &sina, &cosa);
+    glibc_sincosf::sincosf_below_120(cosP * sina, &sC, &cC);
+  }
   p[0] = (float)((double)p[0] + (double)k * ((double)(pxin * sina) - (double)pyin * (1. - (double)cosa)));
   p[1] = (float)((double)p[1] + (double)k * ((double)(pyin * sina) + (double)pxin * (1. - (double)cosa)));
   p[2] = zout;
   p[4] = p[4] + alpha;
-
-  float sC, cC;
-  sincosf_glibc(cosP * sina, &sC, &cC);
   const double omcC = 1. - (double)cC;
   const float J02 = cosP * sinT * (sinP * cosa * sC - cosa) * icosT;
   const float J03 = (float)((double)(cosP * sinT * deltaZ * cosa) * (1. - (double)(sinP * sC)) * (double)(icosT * pt)
@@ -104,11 +201,12 @@ __device__ inline void propagate_ref(Track& t, float hz) {
   float T0[6], T1[6], T4[6];
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
+    if (kZ0 && c == 2) continue;
     const float p0 = P[S(0, c)], p1 = P[S(1, c)], p2 = P[S(2, c)];
     const float p3 = P[S(3, c)], p4 = P[S(4, c)], p5 = P[S(5, c)];
-    T0[c] = p0 + J02 * p2 + J03 * p3 + J04 * p4 + J05 * p5;
-    T1[c] = p1 + J12 * p2 + J13 * p3 + J14 * p4 + J15 * p5;
-    T4[c] = J42 * p2 + J43 * p3 + p4 + J45 * p5;
+    T0[c] = (kZ0 ? p0 : p0 + J02 * p2) + J03 * p3 + J04 * p4 + J05 * p5;
+    T1[c] = (kZ0 ? p1 : p1 + J12 * p2) + J13 * p3 + J14 * p4 + J15 * p5;
+    T4[c] = (kZ0 ? J43 * p3 : J42 * p2 + J43 * p3) + p4 + J45 * p5;
   }
   float T3[6], T5[6];
 #pragma unroll
@@ -118,31 +216,39 @@ __device__ inline void propagate_ref(Track& t, float hz) {
   }
   // P' = T Jt^T.  Entries (2,0) and (2,1) are sums over the zero row of T:
   // they are 0, or NaN when a Jacobian entry is not finite, as in the reference.
-  const float z0 = 0.f;
-  P[S(0, 0)] = T0[0] + T0[2] * J02 + T0[3] * J03 + T0[4] * J04 + T0[5] * J05;
-  P[S(1, 0)] = T1[0] + T1[2] * J02 + T1[3] * J03 + T1[4] * J04 + T1[5] * J05;
-  P[S(1, 1)] = T1[1] + T1[2] * J12 + T1[3] * J13 + T1[4] * J14 + T1[5] * J15;
-  P[S(2, 0)] = z0 + z0 * J02 + z0 * J03 + z0 * J04 + z0 * J05;
-  P[S(2, 1)] = z0 + z0 * J12 + z0 * J13 + z0 * J14 + z0 * J15;
-  P[S(2, 2)] = 0.f;
-  P[S(3, 0)] = T3[0] + T3[2] * J02 + T3[3] * J03 + T3[4] * J04 + T3[5] * J05;
-  P[S(3, 1)] = T3[1] + T3[2] * J12 + T3[3] * J13 + T3[4] * J14 + T3[5] * J15;
-  P[S(3, 2)] = 0.f;
+  auto row0 = [&](const float* T) { return (kZ0 ? T[0] : T[0] + T[2] * J02) + T[3] * J03 + T[4] * J04 + T[5] * J05; };
+  auto row1 = [&](const float* T) { return (kZ0 ? T[1] : T[1] + T[2] * J12) + T[3] * J13 + T[4] * J14 + T[5] * J15; };
+  auto row4 = [&](const float* T) { return (kZ0 ? T[3] * J43 : T[2] * J42 + T[3] * J43) + T[4] + T[5] * J45; };
+  P[S(0, 0)] = row0(T0);
+  P[S(1, 0)] = row0(T1);
+  P[S(1, 1)] = row1(T1);
+  P[S(3, 0)] = row0(T3);
+  P[S(3, 1)] = row1(T3);
   P[S(3, 3)] = T3[3];
-  P[S(4, 0)] = T4[0] + T4[2] * J02 + T4[3] * J03 + T4[4] * J04 + T4[5] * J05;
-  P[S(4, 1)] = T4[1] + T4[2] * J12 + T4[3] * J13 + T4[4] * J14 + T4[5] * J15;
-  P[S(4, 2)] = 0.f;
+  P[S(4, 0)] = row0(T4);
+  P[S(4, 1)] = row1(T4);
   P[S(4, 3)] = T4[3];
-  P[S(4, 4)] = T4[2] * J42 + T4[3] * J43 + T4[4] + T4[5] * J45;
-  P[S(5, 0)] = T5[0] + T5[2] * J02 + T5[3] * J03 + T5[4] * J04 + T5[5] * J05;
-  P[S(5, 1)] = T5[1] + T5[2] * J12 + T5[3] * J13 + T5[4] * J14 + T5[5] * J15;
-  P[S(5, 2)] = 0.f;
+  P[S(4, 4)] = row4(T4);
+  P[S(5, 0)] = row0(T5);
+  P[S(5, 1)] = row1(T5);
   P[S(5, 3)] = T5[3];
-  P[S(5, 4)] = T5[2] * J42 + T5[3] * J43 + T5[4] + T5[5] * J45;
+  P[S(5, 4)] = row4(T5);
   P[S(5, 5)] = T5[5];
+  if constexpr (!kZ0) {
+    const float z0 = 0.f;
+    P[S(2, 0)] = z0 + z0 * J02 + z0 * J03 + z0 * J04 + z0 * J05;
+    P[S(2, 1)] = z0 + z0 * J12 + z0 * J13 + z0 * J14 + z0 * J15;
+  } else {
+    P[S(2, 0)] = P[S(2, 1)] = 0.f;
+  }
+  P[S(2, 2)] = 0.f;
+  P[S(3, 2)] = 0.f;
+  P[S(4, 2)] = 0.f;
+  P[S(5, 2)] = 0.f;
 }
 
-__device__ inline void update_ref(Track& t, const Hit& h) {
+template <bool kZ0>
+__device__ inline void update_ref(Track& t, const Hit& h, bool& ok) {
 #pragma clang fp contract(off)
   float* p = t.p;
   float* P = t.P;
@@ -150,7 +256,18 @@ __device__ inline void update_ref(Track& t, const Hit& h) {
   float r01 = P[1] + h.xy;
   float r11 = P[2] + h.yy;
   const double det = (double)r00 * (double)r11 - (double)r01 * (double)r01;
-  const float s = (float)(1. / det);
+  float s;
+  if constexpr (kZ0) {
+    s = ref_inv_det(det);
+    const float m = __builtin_fabsf(s);  // s in range implies det in ref_inv_det's
+    ok &= m > 0x1p-119f && m < 0x1p119f;
+  } else {
+    const double m = __builtin_fabs(det);
+    if (__builtin_expect(!(m > 0x1p-120 && m < 0x1p120), 0))
+      s = ref_inv_det_any(det);
+    else
+      s = ref_inv_det(det);
+  }
   const float tmp = s * r11;
   r01 = r01 * -s;
   r11 = s * r00;
@@ -158,6 +275,7 @@ __device__ inline void update_ref(Track& t, const Hit& h) {
   float K0[6], K1[6];
 #pragma unroll
   for (int i = 0; i < 6; ++i) {
+    if (kZ0 && i == 2) continue;
     const float a = P[S(i, 0)], b = P[S(i, 1)];
     K0[i] = a * r00 + b * r01;
     K1[i] = a * r01 + b * r11;
@@ -165,14 +283,63 @@ __device__ inline void update_ref(Track& t, const Hit& h) {
   const float res0 = h.x - p[0];
   const float res1 = h.y - p[1];
 #pragma unroll
-  for (int i = 0; i < 6; ++i) p[i] = p[i] + K0[i] * res0 + K1[i] * res1;
+  for (int i = 0; i < 6; ++i) {
+    if (kZ0 && i == 2) continue;
+    p[i] = p[i] + K0[i] * res0 + K1[i] * res1;
+  }
   float C[21];
 #pragma unroll
   for (int i = 0; i < 6; ++i)
 #pragma unroll
-    for (int j = 0; j <= i; ++j) C[S(i, j)] = K0[i] * P[S(0, j)] + K1[i] * P[S(1, j)];
+    for (int j = 0; j <= i; ++j)
+      if (!kZ0 || (i != 2 && j != 2)) C[S(i, j)] = K0[i] * P[S(0, j)] + K1[i] * P[S(1, j)];
 #pragma unroll
-  for (int e = 0; e < 21; ++e) P[e] = P[e] - C[e];
+  for (int i = 0; i < 6; ++i)
+#pragma unroll
+    for (int j = 0; j <= i; ++j)
+      if (!kZ0 || (i != 2 && j != 2)) P[S(i, j)] = P[S(i, j)] - C[S(i, j)];
+}
+
+__device__ inline RefCarry ref_carry(const Track& t) {
+#pragma clang fp contract(off)
+  RefCarry c;
+  c.k = t.q * kKfact;
+  c.rkd = 1. / (double)c.k;
+  return c;
+}
+
+// One layer in the full form.
+__device__ inline void step_ref_full(Track& t, const Hit& h, const RefCarry& c) {
+  bool unused = true;
+  propagate_ref<false>(t, h.z, c, unused);
+  update_ref<false>(t, h, unused);
+}
+
+// After a full step: whether the short form may follow (z row and column +0,
+// no other entry -0).
+__device__ inline bool ref_z0_holds(const Track& t) {
+  uint32_t z = 0;
+  bool ok = true;
+#pragma unroll
+  for (int i = 0; i < 6; ++i)
+#pragma unroll
+    for (int j = 0; j <= i; ++j) {
+      const uint32_t w = __builtin_bit_cast(uint32_t, t.P[S(i, j)]);
+      if (i == 2 || j == 2)
+        z |= w;
+      else
+        ok &= w != 0x80000000u;
+    }
+  return ok && z == 0;
+}
+
+// Positions and diagonal finite (those of a track that ever met a value that
+// is not stay so).
+__device__ inline bool ref_finite(const Track& t) {
+  const bool p = __builtin_isfinite(t.p[0]) && __builtin_isfinite(t.p[1]);
+  const bool u = __builtin_isfinite(t.P[S(0, 0)]) && __builtin_isfinite(t.P[S(1, 1)]);
+  return p && u && __builtin_isfinite(t.P[S(3, 3)]) && __builtin_isfinite(t.P[S(4, 4)]) &&
+         __builtin_isfinite(t.P[S(5, 5)]);
 }
 
 // ---------------------------------------------------------------------------
@@ -239,16 +406,6 @@ __device__ inline void sincos_accurate(float xf, float* sp, float* cp) {
   const float c = (q & 1) ? sf : cf;
   *sp = (q & 2) ? -s : s;
   *cp = ((q + 1) & 2) ? -c : c;
-}
-
-// 1/x rounded to nearest in all but rare cases: the hardware reciprocal
-// (1 ulp) refined by one Newton step with a fused multiply-add.  Every track
-// of an event shares nearly the same ipt / cos(theta); a biased reciprocal
-// would shift all of them the same way, so the 1-ulp estimate alone is not
-// used.
-__device__ inline float fast_rcp(float x) {
-  const float r = __builtin_amdgcn_rcpf(x);
-  return __builtin_fmaf(r, __builtin_fmaf(-x, r, 1.0f), r);
 }
 
 // a / b through the refined reciprocal plus one residual correction.
@@ -810,15 +967,38 @@ __device__ inline void update_v1_fixed(Track& t, const float hc[6], float hx, fl
 // one layer
 // ---------------------------------------------------------------------------
 
+// What a track carries from layer to layer beside its state: sin/cos of phi
+// and theta (FAST, FP64GAIN), or the reference typing's constants; set up on
+// the first layer.
+template <int kMath>
+struct CarryOf {
+  using type = Trig;
+};
+template <>
+struct CarryOf<kRef> {
+  using type = RefCarry;
+};
+template <int kMath>
+using Carry = typename CarryOf<kMath>::type;
+
 // kFirst: the covariance may still have a non-zero z row (first layer of a
-// track); otherwise the fast forms drop the structurally-zero terms.
-// g: sin/cos of phi and theta carried between the layers of one track
-// (FAST, FP64GAIN); set up on the first layer.
+// track); otherwise the structurally-zero terms are dropped.
 template <int kMath, bool kFirst>
-__device__ inline void layer_step(Track& t, const Hit& h, Trig& g) {
+__device__ inline void layer_step(Track& t, const Hit& h, Carry<kMath>& g) {
   if constexpr (kMath == kRef) {
-    propagate_ref(t, h.z);
-    update_ref(t, h);
+    if constexpr (kFirst) {
+      g = ref_carry(t);
+      step_ref_full(t, h, g);
+      g.redo = !ref_z0_holds(t);
+      // +0 already unless the track is marked
+#pragma unroll
+      for (int i = 0; i < 6; ++i) t.P[S(i, 2)] = 0.f;
+    } else {
+      bool ok = true;
+      propagate_ref<true>(t, h.z, g, ok);
+      update_ref<true>(t, h, ok);
+      g.redo |= !ok;
+    }
   } else if constexpr (kMath == kFast) {
     if constexpr (kFirst) trig_init<false>(t, g);
     const Jac J = helix_core<kFirst>(t, h.z, g);

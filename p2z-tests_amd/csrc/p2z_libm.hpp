@@ -19,7 +19,8 @@
 //                                      sin = y, cos = 1 exactly;
 //   |y| < 120                          quadrant n = round(y * 2/pi) from the
 //                                      integer part of y * 2^24*2/pi plus
-//                                      2^23, shifted down 24 bits;
+//                                      2^23, shifted down 24 bits (here by one
+//                                      rounded addition: same floats);
 //                                      r = fma(-n, pi/2, y);
 //   finite                             Payne-Hanek: the 24-bit significand
 //                                      (shifted by the exponent's low 3 bits)
@@ -56,7 +57,7 @@ constexpr double kC4 = 0x1.99343027bf8c3p-16;
 constexpr double kS1 = -0x1.555545995a603p-3;
 constexpr double kS2 = 0x1.1107605230bc4p-7;
 constexpr double kS3 = -0x1.994eb3774cf24p-13;
-constexpr double kTwoOverPiScaled = 0x1.45F306DC9C883p+23;  // 2/pi * 2^24
+constexpr double kTwoOverPi = 0x1.45F306DC9C883p-1;
 constexpr double kPiOver2 = 0x1.921FB54442D18p0;
 constexpr double kPiOver2To63 = 0x1.921FB54442D18p-62;      // pi * 2^-63
 
@@ -74,14 +75,12 @@ __host__ __device__ inline uint32_t top12(uint32_t bits) { return (bits >> 20) &
 
 // Payne-Hanek reduction of a finite float with |y| >= 120 (bits: its bit
 // pattern): r = the reduced argument, n = the quadrant (the low two bits of
-// round(y * 2/pi)).  Kept out of line: inline, its 64-bit products would add
-// their registers to every layer loop that calls sincosf_glibc, where real
-// arguments never reach it.
+// round(y * 2/pi)).
 struct LargeReduction {
   double r;
   int n;
 };
-__host__ __device__ __attribute__((noinline)) inline LargeReduction reduce_large(uint32_t bits) {
+__host__ __device__ inline LargeReduction reduce_large(uint32_t bits) {
   const uint32_t* w = &kInvPio4[(bits >> 26) & 15u];
   const uint32_t m = ((bits & 0xffffffu) | 0x800000u) << ((bits >> 23) & 7u);
   const uint64_t lo = (uint64_t)m * w[8];
@@ -93,57 +92,97 @@ __host__ __device__ __attribute__((noinline)) inline LargeReduction reduce_large
   return LargeReduction{(double)(int64_t)f * kPiOver2To63, (int)n};
 }
 
+// A double constant in scalar registers.  FP64 instructions take no literal
+// operands; left to itself the compiler keeps such constants in vector
+// register pairs across a layer loop.  The empty asm leaves the value
+// unchanged, and moves out of loops.
+__host__ __device__ inline double scalar(double v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm("" : "+s"(v));
+#endif
+  return v;
+}
+
+// sin r and cos r, rounded to float, of a reduced argument and its quadrant q
+// (only its low two bits count): the polynomials above on |r| (both are
+// exactly odd / even in r under round-to-nearest), then the signs and the swap
+// on the two floats, with which rounding commutes.  s0 flips sin, c0 flips cos,
+// odd q swaps them: glibc's sign table {+1, -1, -1, +1} on r and its second
+// coefficient table (cos negated for quadrants 2, 3) come to
+//   q = 0: (s, c)   1: (c, -s)   2: (-s, -c)   3: (-c, s).
+struct Poly {
+  float s, c;  // sin r with r's sign, cos r
+};
+__host__ __device__ inline Poly sincos_reduced(double r) {
+#pragma clang fp contract(off)
+  const double a = __builtin_fabs(r);
+  const double r2 = a * a;
+  const double r3 = r2 * a;
+  const double r4 = r2 * r2;
+  const double r5 = r3 * r2;
+  const double r6 = r4 * r2;
+  const double sin_a = __builtin_fma(r5, __builtin_fma(r2, scalar(kS3), scalar(kS2)), __builtin_fma(r3, scalar(kS1), a));
+  const double cos_a = __builtin_fma(r6, __builtin_fma(r2, scalar(kC4), scalar(kC3)),
+                                     __builtin_fma(r4, scalar(kC2), __builtin_fma(r2, scalar(kC1), kC0)));
+  const uint32_t sign = (uint32_t)(__builtin_bit_cast(uint64_t, r) >> 32) & 0x80000000u;
+  const uint32_t sb = __builtin_bit_cast(uint32_t, (float)sin_a) | sign;
+  return Poly{__builtin_bit_cast(float, sb), (float)cos_a};
+}
+
+// |y| < 0.75: no reduction.
+__host__ __device__ inline void sincosf_small(float y, float* sp, float* cp) {
+  const Poly p = sincos_reduced((double)y);
+  *sp = p.s;
+  *cp = p.c;
+}
+
+// |y| < 120, without a branch: the ranges below 0.75 are the quadrant 0 of the
+// general reduction (r = fma(-0, pi/2, y) = y), and below 2^-12 the
+// polynomials round to sin y = y and cos y = 1 by themselves.  The quadrant is
+// y * 2/pi rounded to nearest by adding 1.5 * 2^52 (its integer then stands in
+// the sum's low word): where that differs from glibc's rounding of the product
+// truncated to 24 fraction bits, next to odd multiples of pi/4, either
+// quadrant gives the same floats.
+__host__ __device__ inline void sincosf_below_120(float y, float* sp, float* cp) {
+#pragma clang fp contract(off)
+  constexpr double kRound = 0x1.8p52;
+  const double x = (double)y;
+  const double t = __builtin_fma(x, scalar(kTwoOverPi), scalar(kRound));
+  const uint32_t q = (uint32_t)__builtin_bit_cast(uint64_t, t);
+  const Poly p = sincos_reduced(__builtin_fma(-(t - scalar(kRound)), scalar(kPiOver2), x));
+  const uint32_t s = __builtin_bit_cast(uint32_t, (q & 1u) ? p.c : p.s);
+  const uint32_t c = __builtin_bit_cast(uint32_t, (q & 1u) ? p.s : p.c);
+  *sp = __builtin_bit_cast(float, s ^ ((q << 30) & 0x80000000u));
+  *cp = __builtin_bit_cast(float, c ^ (((q << 30) + 0x40000000u) & 0x80000000u));
+}
+
+// Everything else: finite |y| >= 120 through Payne-Hanek, infinity and NaN.
+// Kept out of line: inline, its 64-bit products would add their registers to
+// every layer loop that calls sincosf_glibc, where real arguments never reach
+// it.
+__host__ __device__ __attribute__((noinline)) inline Poly sincosf_large(float y) {
+#pragma clang fp contract(off)
+  const uint32_t bits = __builtin_bit_cast(uint32_t, y);
+  if (top12(bits) >= 0x7f8u) return Poly{y - y, y - y};  // inf or NaN
+  const LargeReduction red = reduce_large(bits);
+  const int sgn = red.n + (int)(bits >> 31);  // glibc's index of the sign table
+  const Poly p = sincos_reduced(red.r);
+  const float fs = ((sgn + 1) & 2) ? -p.s : p.s;
+  const float fc = (sgn & 2) ? -p.c : p.c;
+  return (red.n & 1) ? Poly{fc, fs} : Poly{fs, fc};
+}
+
 }  // namespace glibc_sincosf
 
 // sin(y) and cos(y) with glibc's bits.
 __host__ __device__ inline void sincosf_glibc(float y, float* sp, float* cp) {
-#pragma clang fp contract(off)
   using namespace glibc_sincosf;
-  const uint32_t bits = __builtin_bit_cast(uint32_t, y);
-  const uint32_t top = top12(bits);
-  if (top >= 0x7f8u) {  // inf or NaN
-    *sp = *cp = y - y;
-    return;
+  sincosf_below_120(y, sp, cp);
+  if (!(__builtin_fabsf(y) < 120.0f)) {
+    const Poly p = sincosf_large(y);
+    *sp = p.s;
+    *cp = p.c;
   }
-  if (top < 0x398u) {   // |y| < 2^-12
-    *sp = y;
-    *cp = 1.0f;
-    return;
-  }
-  double r;      // reduced argument, |r| <~ pi/4
-  int quad = 0;  // quadrant: selects sin or cos of r
-  int sgn = 0;   // sign pattern index: bit 0 negates r, bit 1 negates cos r
-  if (top < 0x3f4u) {  // |y| < 0.75: no reduction
-    r = (double)y;
-  } else if (top < 0x42fu) {  // |y| < 120
-    const double x = (double)y;
-    const int n = ((int32_t)(x * kTwoOverPiScaled) + 0x800000) >> 24;
-    r = __builtin_fma(-(double)n, kPiOver2, x);
-    quad = n;
-    sgn = n;
-  } else {
-    const LargeReduction red = reduce_large(bits);
-    r = red.r;
-    quad = red.n;
-    sgn = red.n + (int)(bits >> 31);
-  }
-  // glibc's sign table {+1, -1, -1, +1}, indexed by sgn & 3, applied to r.
-  const double rs = ((sgn + 1) & 2) ? -r : r;
-  const double r2 = r * r;
-  const double r3 = r2 * rs;
-  const double r4 = r2 * r2;
-  const double r5 = r3 * r2;
-  const double r6 = r4 * r2;
-  const double sin_tail = __builtin_fma(r2, kS3, kS2);
-  const double sin_r = __builtin_fma(r5, sin_tail, __builtin_fma(r3, kS1, rs));
-  // glibc's second coefficient table (sign indexes 2, 3) negates every cos
-  // coefficient, which negates the cos polynomial exactly.
-  const double cos_abs = __builtin_fma(r6, __builtin_fma(r2, kC4, kC3),
-                                       __builtin_fma(r4, kC2, __builtin_fma(r2, kC1, kC0)));
-  const double cos_r = (sgn & 2) ? -cos_abs : cos_abs;
-  const float fs = (float)sin_r, fc = (float)cos_r;
-  *sp = (quad & 1) ? fc : fs;
-  *cp = (quad & 1) ? fs : fc;
 }
 
 }  // namespace p2z
