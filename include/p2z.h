@@ -183,12 +183,15 @@ typedef struct {
 
 typedef struct {
   int32_t tracks_per_wg; /* 0: the context's setting                          */
-  int32_t prefetch;      /* hit layers loaded ahead: 1 or 2; 0 = 2             */
+  int32_t prefetch;      /* hit layers loaded ahead: 1 or 2; 0 = 1             */
   int32_t waves_per_cu;  /* persistent grid = CUs * waves_per_cu waves; 0 = 8  */
   int32_t items_per_claim; /* persistent form: work items (64 track slots
                               each) per chunk, 1..64; 0 = 4.  Wave w of the
                               grid computes chunk w first, then takes one
                               chunk per atomic on the queue counter       */
+  /* With P2Z_RAGGED_PERSISTENT and neither waves_per_cu nor items_per_claim
+     set, the library chooses the launch: one wave per item, which the
+     hardware's dispatcher hands out in descriptor order.                      */
 } p2z_ragged_opts;
 
 /* Runs every block of the descriptor table (device memory) through its layers.
@@ -299,7 +302,8 @@ typedef struct {
   int32_t width, math;      /* AoSoA width of the pool, arithmetic mode        */
   int32_t tracks_per_wg, prefetch, waves_per_cu, items_per_claim; /* as p2z_ragged_opts, except
                                items_per_claim 0 = 1: a batch of one event
-                               then runs one work item per wave (latency)  */
+                               then runs one work item per wave (latency);
+                               a resident loop's prefetch 0 = 2            */
   int64_t pool_blocks;      /* MPTRK blocks in trk (W-lane rows of lane_nlayer) */
   int64_t pool_hit_blocks;  /* MPHIT blocks in hit; requests are checked
                                against both (p2z_check_blocks) on submit     */

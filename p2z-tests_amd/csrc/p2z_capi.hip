@@ -477,7 +477,7 @@ static int run_ragged_impl(p2z_ctx* c, const void* trk, const void* hit, void* o
   if (nblocks < 0 || nblocks * (int64_t)width > ((int64_t)1 << 31) - 64)
     return p2z::fail(P2Z_EINVAL, "bad block count %lld", (long long)nblocks);
   if (flags & ~(P2Z_RAGGED_PERSISTENT | P2Z_RAGGED_GRAPH)) return p2z::fail(P2Z_EINVAL, "unknown flags 0x%x", flags);
-  int tpw = c->cfg.tracks_per_wg, prefetch = 2, wpc = 8, claim = p2z::kDefaultClaim;
+  int tpw = c->cfg.tracks_per_wg, prefetch = p2z::kDefaultPrefetch, wpc = 0, claim = 0;
   if (opts) {
     if (opts->tracks_per_wg) {
       if (opts->tracks_per_wg < 64 || opts->tracks_per_wg > 256 || opts->tracks_per_wg % 64)
@@ -500,7 +500,9 @@ static int run_ragged_impl(p2z_ctx* c, const void* trk, const void* hit, void* o
   }
   P2Z_TRY(use_device(c));
   if (nblocks == 0) return P2Z_OK;
-  const bool persistent = flags & P2Z_RAGGED_PERSISTENT;
+  const bool persistent = (flags & P2Z_RAGGED_PERSISTENT) && p2z::use_work_queue(wpc, claim);
+  if (!wpc) wpc = p2z::kDefaultWavesPerCu;
+  if (!claim) claim = p2z::kDefaultClaim;
   int64_t grid = ((int64_t)c->cus * wpc * 64 + tpw - 1) / tpw;
   if (persistent) {
     // no more workgroups than the CUs hold at once

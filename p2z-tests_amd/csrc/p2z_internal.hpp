@@ -67,7 +67,23 @@ constexpr size_t kQueueBytes = (size_t)kQueueStripes * kQueueStride * sizeof(uns
 hipError_t launch_ragged(const float* trk, const float* hit, float* out, const int32_t* lane_nlay,
                          const BlockDesc* blocks, int64_t nblocks, int width, int math, bool persistent,
                          int prefetch, int tpw, int64_t grid, int claim, unsigned* counter, hipStream_t s);
+// Shape of a ragged launch whose caller sets nothing but the form.
+// Layers of hits in flight ahead: 1 (fewer registers, one more wave per SIMD;
+// 500 uneven events, FAST: 194 against 199 us persistent, 187 against 188).
+constexpr int kDefaultPrefetch = 1;
+// Items per claim of a persistent launch.
 constexpr int kDefaultClaim = 4;
+// Waves per CU of a persistent launch.
+constexpr int kDefaultWavesPerCu = 8;
+// Whether a pass that may use the work queue runs on it.  With neither the
+// waves per CU nor the items per claim set the library chooses, and takes one
+// wave per item, handed out in table order by the hardware's dispatcher: a
+// queue wave must wait for the stores of one item before the loads of its next
+// (both count on one in-order counter), and the last claims end unevenly.
+// 500 uneven events, FAST: 187 us against 194 for the queue at its best shape
+// (all the waves that fit, 2 items per claim) and 216 at 8 waves per CU and 4
+// items per claim.
+inline bool use_work_queue(int waves_per_cu, int items_per_claim) { return waves_per_cu > 0 || items_per_claim > 0; }
 // Workgroups of tpw threads of the persistent ragged kernel (width, math,
 // prefetch) that one CU holds at once (0 if the runtime cannot tell).  A
 // persistent grid larger than that many per CU leaves waves that start only

@@ -231,15 +231,15 @@ int launch_batches(p2z_server* sv) {
       P2Z_TRY(slot_reserve(s, nblk));
       gather_longest_first(sv, ids, s.h_desc, nblk);
       const int tpw = o.tracks_per_wg ? o.tracks_per_wg : sv->ctx->cfg.tracks_per_wg;
-      const int wpc = o.waves_per_cu ? o.waves_per_cu : 8;
-      const int pf = o.prefetch ? o.prefetch : 2;
+      const int wpc = o.waves_per_cu ? o.waves_per_cu : p2z::kDefaultWavesPerCu;
+      const int pf = o.prefetch ? o.prefetch : p2z::kDefaultPrefetch;
       int64_t grid = ((int64_t)sv->ctx->cus * wpc * 64 + tpw - 1) / tpw;
       const int per_cu = p2z::ragged_persistent_groups_per_cu(o.width, o.math, pf, tpw);
       if (per_cu > 0) grid = std::min<int64_t>(grid, (int64_t)per_cu * sv->ctx->cus);
       P2Z_HIP_CHECK(
           hipMemcpyAsync(s.d_desc, s.h_desc, nblk * sizeof(p2z_block_desc), hipMemcpyHostToDevice, s.stream));
       P2Z_HIP_CHECK(p2z::launch_ragged(sv->trk, sv->hit, sv->arena_mem, sv->lanes, s.d_desc, nblk, o.width, o.math,
-                                       true, pf, tpw, grid,
+                                       p2z::use_work_queue(o.waves_per_cu, o.items_per_claim), pf, tpw, grid,
                                        o.items_per_claim ? o.items_per_claim : 1, s.counter, s.stream));
       P2Z_HIP_CHECK(hipEventRecord(s.done, s.stream));
       return P2Z_OK;

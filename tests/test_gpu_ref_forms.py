@@ -98,7 +98,7 @@ def test_operands_outside_the_short_form(ctx, name):
         dl, db = ctx.upload(np.full(NB * W, nl, np.int32)), ctx.upload(table.view(np.uint8))
         ctx.h2d(dt, trk)
         for persistent in (True, False):
-            ctx.run_ragged(dt, dh, do, dl, db, NB, W, "ref", persistent=persistent)
+            ctx.run_ragged(dt, dh, do, dl, db, NB, W, "ref", persistent=persistent, waves_per_cu=1)
             assert np.array_equal(ctx.download(do).view(np.uint32), got.view(np.uint32)), persistent
         for b in (dt, dh, do, dl, db):
             b.free()
