@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -30,19 +31,16 @@ int use_device(p2z_ctx* c) {
 
 namespace {
 
-// Device scratch of p2z_summary_device_noalloc: results in the first
-// kNoallocResDoubles doubles, the report kernels' per-workgroup partial sums
-// after them.  A file-scope device array: every GPU the library runs on holds
+// Device scratch of p2z_summary_device_noalloc: the report kernel's
+// per-workgroup partial sums.  A file-scope device array: every GPU the library runs on holds
 // its own copy, at its own address, until the process ends, and every call on
 // that GPU shares it.  Host code never passes the array's name to a kernel or
 // a copy (on the host it is only a stand-in for the symbol); it uses the
 // device address hipGetSymbolAddress returns, fetched once per device when
 // the first context on that device is created.
 constexpr size_t kNoallocDoubles = (size_t)P2Z_SUMMARY_NOALLOC_BYTES / sizeof(double);
-constexpr size_t kNoallocResDoubles = 32;
-static_assert(P2Z_SUMMARY_NOALLOC_MAX_TRACKS ==
-                  (P2Z_SUMMARY_NOALLOC_BYTES / 8 - 32) / 12 * 256,
-              "maximum tracks of the header = partial slots of the scratch x 256 tracks");
+static_assert(P2Z_SUMMARY_NOALLOC_MAX_TRACKS == (P2Z_SUMMARY_NOALLOC_BYTES / 8 - 32) / 12 * 256,
+              "the interface's maximum: 12 doubles per 256 tracks; the kernel writes fewer");
 __device__ __align__(256) double scratch[kNoallocDoubles];
 
 std::mutex g_scratch_mu;
@@ -165,7 +163,16 @@ static int create_impl(p2z_ctx** out, int device, const p2z_opts* opts) {
   if (rc == P2Z_OK) rc = p2z::hip_status(hipEventCreate(&c->t1), "hipEventCreate");
   if (rc == P2Z_OK) rc = noalloc_scratch_init(device);
   if (rc == P2Z_OK) rc = apply_opts(c, opts);
-  if (rc == P2Z_OK) rc = p2z::hip_status(hipMalloc((void**)&c->sum_res, 32 * sizeof(double)), "hipMalloc");
+  if (rc == P2Z_OK) rc = p2z::hip_status(hipMalloc((void**)&c->sum_done, p2z::kSumDoneBytes), "hipMalloc");
+  if (rc == P2Z_OK) rc = p2z::hip_status(hipMemsetAsync(c->sum_done, 0, p2z::kSumDoneBytes, c->stream), "hipMemsetAsync");
+  if (rc == P2Z_OK)
+    rc = p2z::hip_status(hipHostMalloc((void**)&c->sum_host, sizeof(p2z::SummaryResult),
+                                       hipHostMallocCoherent | hipHostMallocMapped),
+                         "hipHostMalloc");
+  if (rc == P2Z_OK) {
+    std::memset(c->sum_host, 0, sizeof(p2z::SummaryResult));
+    rc = p2z::hip_status(hipHostGetDevicePointer((void**)&c->sum_dev, c->sum_host, 0), "hipHostGetDevicePointer");
+  }
   if (rc == P2Z_OK) rc = p2z::hip_status(hipMalloc((void**)&c->counter, p2z::kQueueBytes), "hipMalloc");
   if (rc == P2Z_OK)
     rc = p2z::hip_status(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device),
@@ -188,7 +195,8 @@ int p2z_destroy(p2z_ctx* c) {
   if (c->pipe_in) (void)hipStreamDestroy(c->pipe_in);
   if (c->pipe_out) (void)hipStreamDestroy(c->pipe_out);
   if (c->sum_part) (void)hipFree(c->sum_part);
-  if (c->sum_res) (void)hipFree(c->sum_res);
+  if (c->sum_done) (void)hipFree(c->sum_done);
+  if (c->sum_host) (void)hipHostFree(c->sum_host);
   for (auto& kv : c->graphs) (void)hipGraphExecDestroy(kv.second);
   if (c->counter) (void)hipFree(c->counter);
   if (c->t0) (void)hipEventDestroy(c->t0);
@@ -565,15 +573,27 @@ int summary_args(p2z_ctx* c, const void* out, int64_t nevts, int64_t nb, int32_t
   return P2Z_OK;
 }
 
-// Runs the report kernels with the given scratch, then copies the 18 results
-// to the host and unpacks them.
+// Runs the report kernel with the given scratch, waits for its result in host
+// memory and unpacks it.  The sequence number arrives a few us after the last
+// workgroup, where a copy back and a stream synchronisation take tens; a call
+// queued behind long work stops polling after kSummarySpinSeconds and waits
+// for the stream.
+constexpr double kSummarySpinSeconds = 200e-6;
+
 int summary_run(p2z_ctx* c, const void* out, int64_t nevts, int64_t nb, int32_t width, int64_t ntrks,
-                const float* lasthit, double* part, double* res, p2z_summary* s) {
+                const float* lasthit, double* part, p2z_summary* s) {
+  const uint64_t seq = ++c->sum_seq;
   P2Z_HIP_CHECK(p2z::launch_summary((const float*)out, nevts, nb, width, ntrks, lasthit[0], lasthit[1],
-                                    lasthit[2], part, res, c->stream));
+                                    lasthit[2], part, c->sum_done, c->sum_dev, seq, c->stream));
+  const auto arrived = [&] { return __atomic_load_n(&c->sum_host->seq, __ATOMIC_ACQUIRE) == seq; };
+  const auto t0 = std::chrono::steady_clock::now();
+  while (!arrived()) {
+    if (std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() < kSummarySpinSeconds) continue;
+    P2Z_HIP_CHECK(hipStreamSynchronize(c->stream));
+    if (!arrived()) return p2z::fail(P2Z_EHIP, "the report kernel ended without a result");
+  }
   double r[18];
-  P2Z_HIP_CHECK(hipMemcpyAsync(r, res, sizeof r, hipMemcpyDeviceToHost, c->stream));
-  P2Z_HIP_CHECK(hipStreamSynchronize(c->stream));
+  std::memcpy(r, c->sum_host->bits, sizeof r);
   std::memset(s, 0, sizeof *s);
   s->avgx = r[0]; s->avgy = r[1]; s->avgz = r[2];
   s->avgdx = r[3]; s->avgdy = r[4]; s->avgdz = r[5];
@@ -598,7 +618,7 @@ int p2z_summary_device(p2z_ctx* c, const void* out, int64_t nevts, int64_t nb, i
     P2Z_HIP_CHECK(hipMalloc((void**)&c->sum_part, need * sizeof(double)));
     c->sum_part_len = need;
   }
-  return summary_run(c, out, nevts, nb, width, ntrks, lasthit, c->sum_part, c->sum_res, s);
+  return summary_run(c, out, nevts, nb, width, ntrks, lasthit, c->sum_part, s);
 }
 
 int p2z_summary_device_noalloc(p2z_ctx* c, const void* out, int64_t nevts, int64_t nb, int32_t width,
@@ -610,9 +630,9 @@ int p2z_summary_device_noalloc(p2z_ctx* c, const void* out, int64_t nevts, int64
   P2Z_TRY(use_device(c));
   double* base = noalloc_scratch(c->device);
   if (!base) return p2z::fail(P2Z_ESTATE, "static report scratch of GPU %d not set up", c->device);
-  // every partial slot the kernels read is written first in the same call,
-  // and the results are written before they are read: nothing to clear
-  return summary_run(c, out, nevts, nb, width, ntrks, lasthit, base + kNoallocResDoubles, base, s);
+  // every partial slot the kernel reads is written first in the same call:
+  // nothing to clear
+  return summary_run(c, out, nevts, nb, width, ntrks, lasthit, base, s);
 }
 
 }  // extern "C"

@@ -25,7 +25,10 @@ struct p2z_ctx {
   // device report scratch
   double* sum_part = nullptr;
   size_t sum_part_len = 0;
-  double* sum_res = nullptr;
+  unsigned* sum_done = nullptr;             // workgroups finished (device)
+  p2z::SummaryResult* sum_host = nullptr;   // result in pinned memory, and its device view
+  p2z::SummaryResult* sum_dev = nullptr;
+  uint64_t sum_seq = 0;                     // calls so far
   // ragged path: work-queue counter, compute units, captured graphs
   unsigned* counter = nullptr;
   int cus = 0;

@@ -91,13 +91,24 @@ inline bool use_work_queue(int waves_per_cu, int items_per_claim) { return waves
 // a claim, are then the longest items computed last.
 int ragged_persistent_groups_per_cu(int width, int math, int prefetch, int tpw);
 
-// Report statistics (OMP:758-851) on device.  part: scratch of
-// summary_scratch_doubles(nevts, ntrks) doubles.  res: 18 doubles on device
-// (9 means, 3 counts, 6 RMS values), written by the final passes.
+// Result of the report statistics in host memory (pinned, coherent): 9 means,
+// 3 counts (nnans, nfail, ngood) and 6 RMS values as the bits of doubles, then
+// the call's sequence number, written last.
+struct SummaryResult {
+  uint64_t bits[18];
+  uint64_t seq;
+};
+
+// Report statistics (OMP:758-851) on device, one launch.  part: scratch of
+// summary_scratch_doubles(nevts, ntrks) doubles.  done: kSumDoneBytes of
+// counters in device memory, zero before and after.  res: device view of the result.
+constexpr int kSumStripes = 16;
+constexpr int kSumStride = 32;  // 32-bit words between counters: a 128-byte line each
+constexpr size_t kSumDoneBytes = (size_t)(1 + kSumStripes) * kSumStride * sizeof(unsigned);
 size_t summary_scratch_doubles(int64_t nevts, int64_t ntrks);
 hipError_t launch_summary(const float* out, int64_t nevts, int64_t nb, int width, int64_t ntrks,
-                          double hx, double hy, double hz, double* part, double* res,
-                          hipStream_t s);
+                          double hx, double hy, double hz, double* part, unsigned* done, SummaryResult* res,
+                          uint64_t seq, hipStream_t s);
 
 // ---- device-resident serving loop -------------------------------------------
 // Work item of the resident loop: 64 track slots of one request.  W <= 64:

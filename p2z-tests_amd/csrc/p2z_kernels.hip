@@ -616,125 +616,220 @@ __global__ __launch_bounds__(256) void k_update_v1(float* trkErr, float* inPar, 
 // ---------------------------------------------------------------------------
 // report statistics (OMP:758-851), deterministic fixed-order reduction
 // ---------------------------------------------------------------------------
+// One launch over the tracks.  A workgroup takes kSumTracks tracks per thread,
+// sums them, forms the means of its own tracks and, from the values still in
+// registers, the sums of squares about those means; its partial results go to
+// memory.  The workgroup that finishes last combines the partials in their
+// fixed order: means from the sums, then
+//   sum (x - mean)^2 = sum over workgroups of M2 + n (mean of the workgroup - mean)^2,
+// whose terms are all positive, so it is as accurate as the reference's second
+// pass over the tracks without one.  It writes the result into host memory
+// with a sequence number behind it, which the host waits for.
+// Bound: latency.  960000 tracks (23 MB read): 75 us per call as two passes
+// over the tracks, two final launches and a copy back; 28 us now (20 us of it
+// the kernel: loads, the divisions in double, four sums over a workgroup, the
+// last of which nothing overlaps; 4 or 2 tracks per thread: 29 and 33 us).
 constexpr int kSumThreads = 256;
-constexpr int kSumVals = 12;  // pass 1: 9 sums + nnans, nfail, ngood; pass 2: 6 sums
+constexpr int kSumTracks = 8;
+constexpr int kSumMeans = 9;  // x y z dx dy dz pt phi theta
+constexpr int kSumRms = 6;    // x y z dx dy dz
+constexpr int kSumVals = kSumMeans + kSumRms + 3;  // sums, squares about the workgroup's means, counts
 
-struct TrackView {
-  double x, y, z, pt, phi, theta;
-  int state;  // 0 good, 1 non-finite, 2 outside the acceptance window
-};
-
-__device__ inline TrackView view_track(const float* out, int64_t nb, int W, int64_t ntrks,
-                                       int64_t idx, double hx, double hy, double hz) {
-  const int64_t ie = idx / ntrks, it = idx % ntrks;
-  const float* blk = out + ((it / W) + nb * ie) * (int64_t)(kTrkWords * W);
-  const int64_t l = it % W;
-  TrackView v;
-  v.x = blk[0 * W + l];
-  v.y = blk[1 * W + l];
-  v.z = blk[2 * W + l];
-  v.pt = 1. / (double)blk[3 * W + l];
-  v.phi = blk[4 * W + l];
-  v.theta = blk[5 * W + l];
-  if (!isfinite(v.x) || !isfinite(v.y) || !isfinite(v.z) || !isfinite(v.pt) ||
-      !isfinite(v.phi) || !isfinite(v.theta)) {
-    v.state = 1;
-  } else if (fabs((v.x - hx) / hx) > 1. || fabs((v.y - hy) / hy) > 1. ||
-             fabs((v.z - hz) / hz) > 1. || fabs((v.pt - 12.) / 12.) > 1. ||
-             fabs((v.phi - 1.3) / 1.3) > 1. || fabs((v.theta - 2.8) / 2.8) > 1.) {
-    v.state = 2;
-  } else {
-    v.state = 0;
-  }
-  return v;
+// Sum over each row of 16 lanes, the same in all of them (all active).
+template <int kCtrl>
+__device__ inline double add_dpp(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, kCtrl, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), kCtrl, 0xf, 0xf, true);
+  return v + __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ inline double row_sum(double v) {
+  v = add_dpp<0xB1>(v);     // lanes 1 0 3 2 of each four
+  v = add_dpp<0x4E>(v);     // lanes 2 3 0 1
+  v = add_dpp<0x141>(v);    // mirrored within 8
+  return add_dpp<0x140>(v); // mirrored within 16
 }
 
-// Tree-reduce kSumVals doubles per thread over the workgroup in a fixed order;
-// thread 0 returns the totals in vals.
-__device__ inline void block_reduce(double (&vals)[kSumVals], double* lds) {
+// Adds v over the workgroup; every thread gets the totals.  The values go
+// through LDS once, 16 threads then add up each: 60 instructions per thread
+// for 12 values, where a butterfly of shuffles takes 140 LDS operations and
+// one of data-parallel primitives 280 instructions.
+constexpr int kSumRow = kSumThreads + 16;  // padded: rows of 16 threads read different banks
+struct SumLds {
+  double v[(kSumMeans + 3) * kSumRow];
+  double total[kSumMeans + 3];
+};
+template <int kN>
+__device__ inline void block_sum(double (&v)[kN], SumLds& lds) {
   const int t = threadIdx.x;
 #pragma unroll
-  for (int k = 0; k < kSumVals; ++k) lds[k * kSumThreads + t] = vals[k];
+  for (int k = 0; k < kN; ++k) lds.v[k * kSumRow + t] = v[k];
   __syncthreads();
-  for (int stride = kSumThreads / 2; stride > 0; stride >>= 1) {
-    if (t < stride) {
+  const int k0 = t / 16;
+  if (k0 < kN) {  // whole rows of 16 lanes
+    double s = 0.;
 #pragma unroll
-      for (int k = 0; k < kSumVals; ++k) lds[k * kSumThreads + t] += lds[k * kSumThreads + t + stride];
-    }
-    __syncthreads();
+    for (int i = 0; i < 16; ++i) s += lds.v[k0 * kSumRow + i * 16 + t % 16];
+    s = row_sum(s);
+    if (t % 16 == 0) lds.total[k0] = s;
   }
+  __syncthreads();
 #pragma unroll
-  for (int k = 0; k < kSumVals; ++k) vals[k] = lds[k * kSumThreads];
+  for (int k = 0; k < kN; ++k) v[k] = lds.total[k];
+  __syncthreads();
 }
 
-template <int W, int kPass>
-__global__ __launch_bounds__(kSumThreads) void k_summary(const float* __restrict__ out, int64_t nb,
-                                                         int64_t ntrks, int64_t total, double hx,
-                                                         double hy, double hz,
-                                                         const double* __restrict__ res,
-                                                         double* __restrict__ part) {
-  __shared__ double lds[kSumVals * kSumThreads];
-  double v[kSumVals];
+// Counts the caller in; true for the last of n, which sets the counter back.
+__device__ inline bool last_of(unsigned* counter, unsigned n) {
+  if (__hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u != n) return false;
+  __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+template <int W>
+__global__ __launch_bounds__(kSumThreads) void k_summary(const float* __restrict__ out, int64_t nb, int64_t ntrks,
+                                                         int64_t total, double hx, double hy, double hz,
+                                                         double* part, unsigned* done, SummaryResult* res,
+                                                         uint64_t seq) {
+  __shared__ SumLds lds;
+  __shared__ double own[kSumVals];
+  __shared__ unsigned last;
+  // a thread's tracks are kSumThreads apart, all their words loaded at once
+  const int64_t idx0 = (int64_t)blockIdx.x * (kSumThreads * kSumTracks) + threadIdx.x;
+  int64_t ie, it;
+  if (total < (int64_t)1 << 31) {  // a 64-bit division takes a hundred instructions
+    ie = (uint32_t)idx0 / (uint32_t)ntrks;
+    it = (uint32_t)idx0 % (uint32_t)ntrks;
+  } else {
+    ie = idx0 / ntrks;
+    it = idx0 % ntrks;
+  }
+  float w[kSumTracks][6];
 #pragma unroll
-  for (int k = 0; k < kSumVals; ++k) v[k] = 0.;
-  const int64_t idx = (int64_t)blockIdx.x * kSumThreads + threadIdx.x;
-  if (idx < total) {
-    const TrackView tv = view_track(out, nb, W, ntrks, idx, hx, hy, hz);
-    if (kPass == 1) {
-      if (tv.state == 0) {
-        v[0] = tv.x; v[1] = tv.y; v[2] = tv.z;
-        v[3] = (tv.x - hx) / tv.x; v[4] = (tv.y - hy) / tv.y; v[5] = (tv.z - hz) / tv.z;
-        v[6] = tv.pt; v[7] = tv.phi; v[8] = tv.theta;
-        v[11] = 1.;
-      } else if (tv.state == 1) {
-        v[9] = 1.;
+  for (int k = 0; k < kSumTracks; ++k) {
+    if (idx0 + k * kSumThreads < total) {
+      const float* blk = out + ((it / W) + nb * ie) * (int64_t)(kTrkWords * W) + it % W;
+#pragma unroll
+      for (int e = 0; e < 6; ++e) w[k][e] = blk[e * W];
+    }
+    it += kSumThreads;
+    if (it >= ntrks) {
+      if (it < 2 * ntrks) {
+        it -= ntrks;
+        ++ie;
       } else {
-        v[10] = 1.;
+        ie += it / ntrks;
+        it %= ntrks;
       }
-    } else if (tv.state == 0) {
-      const double dx = tv.x - res[0], dy = tv.y - res[1], dz = tv.z - res[2];
-      const double ddx = (tv.x - hx) / tv.x - res[3], ddy = (tv.y - hy) / tv.y - res[4],
-                   ddz = (tv.z - hz) / tv.z - res[5];
-      v[0] = dx * dx; v[1] = dy * dy; v[2] = dz * dz;
-      v[3] = ddx * ddx; v[4] = ddy * ddy; v[5] = ddz * ddz;
     }
   }
-  block_reduce(v, lds);
+  double x[kSumTracks][kSumRms];
+  bool good[kSumTracks];
+  double v[kSumMeans + 3];  // sums of the means' values, then nnans, nfail, ngood
+#pragma unroll
+  for (int k = 0; k < kSumMeans + 3; ++k) v[k] = 0.;
+#pragma unroll
+  for (int k = 0; k < kSumTracks; ++k) {
+    good[k] = false;
+    if (idx0 + k * kSumThreads < total) {
+      const double X = w[k][0], Y = w[k][1], Z = w[k][2], ipt = w[k][3], phi = w[k][4], theta = w[k][5];
+      const double pt = 1. / ipt;
+      if (!isfinite(X) || !isfinite(Y) || !isfinite(Z) || !isfinite(pt) || !isfinite(phi) || !isfinite(theta)) {
+        v[kSumMeans] += 1.;
+      } else if (fabs(X - hx) > fabs(hx) || fabs(Y - hy) > fabs(hy) || fabs(Z - hz) > fabs(hz) ||
+                 fabs(pt - 12.) > 12. || fabs(phi - 1.3) > 1.3 || fabs(theta - 2.8) > 2.8) {
+        // the window |(x - hx) / hx| > 1 without its division: a quotient of
+        // doubles rounds above 1 exactly when the numerator is the larger
+        v[kSumMeans + 1] += 1.;
+      } else {
+        good[k] = true;
+        x[k][0] = X;
+        x[k][1] = Y;
+        x[k][2] = Z;
+        x[k][3] = (X - hx) / X;
+        x[k][4] = (Y - hy) / Y;
+        x[k][5] = (Z - hz) / Z;
+#pragma unroll
+        for (int e = 0; e < kSumRms; ++e) v[e] += x[k][e];
+        v[6] += pt;
+        v[7] += phi;
+        v[8] += theta;
+        v[kSumMeans + 2] += 1.;
+      }
+    }
+  }
+  block_sum(v, lds);
+  double m2[kSumRms];
+  const double n = v[kSumMeans + 2];
+#pragma unroll
+  for (int e = 0; e < kSumRms; ++e) {
+    const double mean = n > 0. ? v[e] / n : 0.;
+    m2[e] = 0.;
+#pragma unroll
+    for (int k = 0; k < kSumTracks; ++k)
+      if (good[k]) m2[e] += (x[k][e] - mean) * (x[k][e] - mean);
+  }
+  block_sum(m2, lds);
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int k = 0; k < kSumVals; ++k) part[(int64_t)blockIdx.x * kSumVals + k] = v[k];
+    for (int k = 0; k < kSumMeans + 3; ++k) own[k] = v[k];
+#pragma unroll
+    for (int e = 0; e < kSumRms; ++e) own[kSumMeans + 3 + e] = m2[e];
   }
-}
+  if (threadIdx.x < 64) {
+    // one store instruction for the partials, written through to where every
+    // XCD sees them, and complete before the workgroup is counted
+    if (threadIdx.x < kSumVals)
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(part + (int64_t)blockIdx.x * kSumVals) + threadIdx.x,
+                         __builtin_bit_cast(uint64_t, own[threadIdx.x]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    wait_stores();
+  }
+  if (threadIdx.x == 0) {
+    // counted in two steps: one counter for all workgroups would take them one
+    // after another (about 15 ns each)
+    const unsigned ns = gridDim.x < (unsigned)kSumStripes ? gridDim.x : kSumStripes;
+    const unsigned stripe = blockIdx.x % ns;
+    last = last_of(done + (1 + stripe) * kSumStride, (gridDim.x - stripe + ns - 1) / ns) && last_of(done, ns);
+  }
+  __syncthreads();
+  if (!last) return;
 
-// Final reduction of the per-workgroup partials (one workgroup).  Pass 1 turns
-// the sums into means (res[0..8]) and counts (res[9..11] = nnans, nfail, ngood);
-// pass 2 into the rounded-to-float RMS values (res[12..17]).
-template <int kPass>
-__global__ __launch_bounds__(kSumThreads) void k_summary_final(const double* __restrict__ part,
-                                                               int64_t nparts,
-                                                               double* __restrict__ res) {
-  __shared__ double lds[kSumVals * kSumThreads];
-  double v[kSumVals];
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // no partial is read from a cache filled before
+  const int64_t groups = gridDim.x;
 #pragma unroll
-  for (int k = 0; k < kSumVals; ++k) v[k] = 0.;
-  for (int64_t i = threadIdx.x; i < nparts; i += kSumThreads) {
+  for (int k = 0; k < kSumMeans + 3; ++k) v[k] = 0.;
+  for (int64_t g = threadIdx.x; g < groups; g += kSumThreads) {
 #pragma unroll
-    for (int k = 0; k < kSumVals; ++k) v[k] += part[i * kSumVals + k];
+    for (int k = 0; k < kSumMeans + 3; ++k) v[k] += part[g * kSumVals + k];
   }
-  block_reduce(v, lds);
-  if (threadIdx.x == 0) {
-    if (kPass == 1) {
-      const double n = v[11];
+  block_sum(v, lds);
+  const double ngood = v[kSumMeans + 2];
 #pragma unroll
-      for (int k = 0; k < 9; ++k) res[k] = v[k] / n;
-      res[9] = v[9];
-      res[10] = v[10];
-      res[11] = v[11];
-    } else {
-      const double n = res[11];
+  for (int e = 0; e < kSumRms; ++e) m2[e] = 0.;
+  for (int64_t g = threadIdx.x; g < groups; g += kSumThreads) {
+    const double* p = part + g * kSumVals;
+    const double ng = p[kSumMeans + 2];
+    if (ng > 0.) {
 #pragma unroll
-      for (int k = 0; k < 6; ++k) res[12 + k] = (double)sqrtf((float)(v[k] / n));
+      for (int e = 0; e < kSumRms; ++e) {
+        const double d = p[e] / ng - v[e] / ngood;
+        m2[e] += p[kSumMeans + 3 + e] + ng * (d * d);
+      }
     }
+  }
+  block_sum(m2, lds);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < kSumMeans; ++k) own[k] = v[k] / ngood;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) own[kSumMeans + k] = v[kSumMeans + k];
+#pragma unroll
+    for (int e = 0; e < kSumRms; ++e) own[kSumMeans + 3 + e] = (double)sqrtf((float)(m2[e] / ngood));
+  }
+  if (threadIdx.x < 64) {
+    if (threadIdx.x < kSumVals) sys_store(&res->bits[threadIdx.x], __builtin_bit_cast(uint64_t, own[threadIdx.x]));
+    wait_stores();
+    if (threadIdx.x == 0) sys_store(&res->seq, seq);
   }
 }
 
@@ -930,23 +1025,19 @@ hipError_t launch_sincosf_range(uint32_t first, int64_t n, float* s, float* c, h
 }
 
 size_t summary_scratch_doubles(int64_t nevts, int64_t ntrks) {
-  return (size_t)grid_for(nevts * ntrks, kSumThreads) * kSumVals;
+  return (size_t)grid_for(nevts * ntrks, kSumThreads * kSumTracks) * kSumVals;
 }
 
 hipError_t launch_summary(const float* out, int64_t nevts, int64_t nb, int width, int64_t ntrks,
-                          double hx, double hy, double hz, double* part, double* res,
-                          hipStream_t s) {
+                          double hx, double hy, double hz, double* part, unsigned* done, SummaryResult* res,
+                          uint64_t seq, hipStream_t s) {
   const int64_t total = nevts * ntrks;
-  const int64_t nparts = grid_for(total, kSumThreads);
-  if (nparts == 0) return hipErrorInvalidValue;
+  const int64_t groups = grid_for(total, kSumThreads * kSumTracks);
+  if (groups == 0) return hipErrorInvalidValue;
   return dispatch_width(width, [&](auto wc) {
     constexpr int W = decltype(wc)::value;
-    hipLaunchKernelGGL((k_summary<W, 1>), dim3((unsigned)nparts), dim3(kSumThreads), 0, s, out, nb,
-                       ntrks, total, hx, hy, hz, res, part);
-    hipLaunchKernelGGL((k_summary_final<1>), dim3(1), dim3(kSumThreads), 0, s, part, nparts, res);
-    hipLaunchKernelGGL((k_summary<W, 2>), dim3((unsigned)nparts), dim3(kSumThreads), 0, s, out, nb,
-                       ntrks, total, hx, hy, hz, res, part);
-    hipLaunchKernelGGL((k_summary_final<2>), dim3(1), dim3(kSumThreads), 0, s, part, nparts, res);
+    hipLaunchKernelGGL((k_summary<W>), dim3((unsigned)groups), dim3(kSumThreads), 0, s, out, nb, ntrks, total, hx, hy,
+                       hz, part, done, res, seq);
     return hipGetLastError();
   });
 }
