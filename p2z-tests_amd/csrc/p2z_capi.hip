@@ -83,6 +83,10 @@ void free_pipeline_slots(p2z_ctx* c) {
   c->pipe.clear();
   c->slot_trk.clear(); c->slot_hit.clear(); c->slot_out.clear();
   c->slot_trk_bytes = c->slot_hit_bytes = 0;
+  for (auto p : c->stage_in) (void)hipHostFree(p);
+  for (auto p : c->stage_out) (void)hipHostFree(p);
+  c->stage_in.clear(); c->stage_out.clear();
+  c->stage_in_bytes = c->stage_out_bytes = 0;
 }
 
 int apply_opts(p2z_ctx* c, const p2z_opts* o) {
@@ -372,41 +376,78 @@ int p2z_sincosf_ref(p2z_ctx* c, uint32_t first_bits, int64_t n, float* s, float*
 
 namespace {
 
-// True for page-locked host memory (hipHostMalloc); pageable memory makes
-// hipPointerGetAttributes fail or report unregistered memory.
-bool host_pinned(const void* p) {
+// Where a caller's buffer lies: page-locked host memory (hipHostMalloc), plain
+// pageable memory (unknown to the runtime), or anything else it knows.
+enum class Where { kPinned, kPageable, kOther };
+Where where_is(const void* p) {
   hipPointerAttribute_t a;
   if (hipPointerGetAttributes(&a, p) != hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return Where::kPageable;
   }
-  return a.type == hipMemoryTypeHost;
+  if (a.type == hipMemoryTypeHost) return Where::kPinned;
+  return a.type == hipMemoryTypeUnregistered ? Where::kPageable : Where::kOther;
+}
+
+// Grows a set of n pinned buffers to `bytes` each.
+int stage_reserve(std::vector<char*>& bufs, size_t& have, int n, size_t bytes) {
+  if (have >= bytes && (int)bufs.size() == n) return P2Z_OK;
+  for (auto p : bufs) (void)hipHostFree(p);
+  bufs.assign(n, nullptr);
+  have = 0;
+  for (auto& p : bufs) {
+    const hipError_t e = hipHostMalloc((void**)&p, bytes, hipHostMallocDefault);
+    if (e == hipErrorOutOfMemory) return p2z::fail(P2Z_ENOMEM, "pinned staging buffers do not fit");
+    P2Z_HIP_CHECK(e);
+  }
+  have = bytes;
+  return P2Z_OK;
 }
 
 }  // namespace
 
+// Blocks go through ns staging slots in chunks, in three stages: every copy in
+// runs on pipe_in, one after another at the full PCIe rate (copies in on
+// several streams would share the link and reach their kernels, then their
+// copies out, at the same time, leaving the link idle while they drain); chunk
+// k's kernel runs on slot k % ns's stream; every copy out runs on pipe_out,
+// beside the copies in.  A device slot is reused once its previous kernel has
+// read the inputs (ev_done) and its previous output has been copied out
+// (ev_out).
+// Pageable buffers are staged here through pinned slots by several threads,
+// only the hit words the path reads (the runtime's own staging is one thread:
+// 10 events x 9600 x 20, 80 MB of buffers, 4.3 ms, now 1.38; 100 events 34 and
+// 12 ms; from pinned buffers 1.22 and 10.8).  A pinned slot is refilled once
+// its copies in have run (ev_in), and emptied before its chunk's slot comes
+// round again.
 static int run_host_impl(p2z_ctx* c, const void* trk, const void* hit, void* out, int64_t nevts, int64_t nb,
                          int32_t nlayer, int32_t width, int32_t math) {
   if (!c) return p2z::fail(P2Z_EINVAL, "null ctx");
   P2Z_TRY(check_blocks(trk, hit, out, nevts, nb, nlayer, width, math));
   P2Z_TRY(use_device(c));
-  if (nevts == 0 || nb == 0) return P2Z_OK;
+  const int64_t nblocks = nevts * nb;
+  if (nblocks == 0) return P2Z_OK;
   const int ns = (int)c->pipe.size();
-  const bool hit_pinned = nlayer > 0 && host_pinned(hit);
-  // Chunks of whole events through ns staging slots, in three stages: every
-  // copy in runs on pipe_in, one after another at the full PCIe rate (copies
-  // in on several streams would share the link and reach their kernels, then
-  // their copies out, at the same time, leaving the link idle while they
-  // drain); chunk k's kernel runs on slot k % ns's stream; every copy out runs
-  // on pipe_out, beside the copies in.  Four chunks per slot keep the last
-  // kernel and copy out, which nothing overlaps, short.  A slot is reused once
-  // its previous kernel has read the inputs (ev_done) and its previous output
-  // has been copied out (ev_out).
-  const int64_t nchunks = std::min<int64_t>(nevts, 4 * (int64_t)ns);
-  const int64_t per = (nevts + nchunks - 1) / nchunks;
-  const size_t trk_ev = (size_t)nb * p2z::kTrkWords * width * sizeof(float);
-  const size_t hit_ev = (size_t)nb * nlayer * p2z::kHitWords * width * sizeof(float);
-  const size_t need_trk = trk_ev * per, need_hit = std::max<size_t>(hit_ev * per, 1);
+  const Where hit_at = nlayer > 0 ? where_is(hit) : Where::kOther;
+  const bool stage_trk = where_is(trk) == Where::kPageable, stage_hit = hit_at == Where::kPageable;
+  const bool stage_dst = where_is(out) == Where::kPageable;
+  const size_t trk_blk = (size_t)p2z::kTrkWords * width * sizeof(float);
+  const size_t hit_rec = (size_t)p2z::kHitWords * width * sizeof(float);
+  const size_t hit_used = (size_t)p2z::kHitUsedWords * width * sizeof(float);
+  const size_t hit_blk = hit_rec * nlayer;
+  // Three chunks per slot keep the last kernel and copy out, which nothing
+  // overlaps, short.  No chunk below kMinChunk bytes of input where more
+  // than one is made: each costs about 40 us of its own on the link (10 events,
+  // 80 MB, pinned: 10 chunks 1.48 ms, 5 1.28, 3 1.19).  Staged chunks are no
+  // larger than that (kept pinned memory, and the first one's staging is not
+  // overlapped; 10 events: 16 MB 1.49 ms, 32 MB 1.41).
+  constexpr size_t kMinChunk = 32 << 20;
+  const size_t total = (size_t)nblocks * (trk_blk + hit_blk);
+  const size_t want = stage_hit || stage_trk ? kMinChunk : std::max(kMinChunk, total / (3 * (size_t)ns));
+  const int64_t most = (int64_t)std::min<size_t>((size_t)nblocks, (total + want - 1) / want);
+  const int64_t per = (nblocks + most - 1) / most;
+  const int64_t nchunks = (nblocks + per - 1) / per;
+  const size_t need_trk = trk_blk * per, need_hit = std::max<size_t>(hit_blk * per, 1);
   if (c->slot_trk_bytes < need_trk || c->slot_hit_bytes < need_hit || (int)c->slot_trk.size() != ns) {
     P2Z_HIP_CHECK(sync_pipeline(c));
     for (auto p : c->slot_trk) (void)hipFree(p);
@@ -424,44 +465,63 @@ static int run_host_impl(p2z_ctx* c, const void* trk, const void* hit, void* out
     c->slot_trk_bytes = need_trk;
     c->slot_hit_bytes = need_hit;
   }
+  const size_t in_hit = stage_trk ? need_trk : 0;  // offset of the hits in a pinned slot
+  if (stage_trk || stage_hit)
+    P2Z_TRY(stage_reserve(c->stage_in, c->stage_in_bytes, ns,
+                          in_hit + (stage_hit ? hit_used * (size_t)nlayer * per : 0)));
+  if ((stage_trk || stage_hit || stage_dst) && !c->copy) c->copy = std::make_unique<p2z::CopyPool>();
+  if (stage_dst) P2Z_TRY(stage_reserve(c->stage_out, c->stage_out_bytes, ns, need_trk));
+  // the result of chunk k from its pinned slot to the caller's buffer
+  const auto drain = [&](int64_t k) -> int {
+    const int64_t b0 = k * per, n = std::min(nblocks, b0 + per) - b0;
+    P2Z_HIP_CHECK(hipEventSynchronize(c->ev_out[k % ns]));
+    c->copy->rows((char*)out + b0 * trk_blk, trk_blk, c->stage_out[k % ns], trk_blk, trk_blk, (size_t)n);
+    return P2Z_OK;
+  };
   // every path out waits for the pipeline streams: no copy from or to the
   // caller's host buffers is still in flight when this returns
   const int rc = [&]() -> int {
     for (int64_t k = 0; k < nchunks; ++k) {
-      const int64_t e0 = k * per, e1 = std::min(nevts, e0 + per);
-      if (e0 >= e1) break;
+      const int64_t b0 = k * per, n = std::min(nblocks, b0 + per) - b0;
       const int i = (int)(k % ns);
       const bool reuse = k >= ns;  // slot i held chunk k - ns
-      const int64_t ne = e1 - e0;
+      const char* src_trk = (const char*)trk + b0 * trk_blk;
+      const char* src_hit = (const char*)hit + b0 * hit_blk;
       if (reuse) P2Z_HIP_CHECK(hipStreamWaitEvent(c->pipe_in, c->ev_done[i], 0));
-      P2Z_HIP_CHECK(hipMemcpyAsync(c->slot_trk[i], (const char*)trk + e0 * trk_ev, ne * trk_ev,
-                                   hipMemcpyHostToDevice, c->pipe_in));
-      if (hit_pinned) {
+      if (reuse && (stage_trk || stage_hit)) P2Z_HIP_CHECK(hipEventSynchronize(c->ev_in[i]));
+      if (stage_trk) {
+        c->copy->rows(c->stage_in[i], trk_blk, src_trk, trk_blk, trk_blk, (size_t)n);
+        src_trk = c->stage_in[i];
+      }
+      P2Z_HIP_CHECK(hipMemcpyAsync(c->slot_trk[i], src_trk, n * trk_blk, hipMemcpyHostToDevice, c->pipe_in));
+      if (stage_hit) {
+        c->copy->rows(c->stage_in[i] + in_hit, hit_used, src_hit, hit_rec, hit_used, (size_t)(n * nlayer));
+        src_hit = c->stage_in[i] + in_hit;
+      }
+      if (stage_hit || hit_at == Where::kPinned) {
         // only the words the path reads: pos x, y, z and cov xx, xy, yy of each
         // hit record (the record's last 3W words, cov xz, yz, zz, are never
-        // read, OMP:510-512); one row per record, same pitch on both sides
-        const size_t pitch = (size_t)p2z::kHitWords * width * sizeof(float);
-        P2Z_HIP_CHECK(hipMemcpy2DAsync(c->slot_hit[i], pitch, (const char*)hit + e0 * hit_ev, pitch,
-                                       (size_t)p2z::kHitUsedWords * width * sizeof(float),
-                                       (size_t)(ne * nb * nlayer), hipMemcpyHostToDevice, c->pipe_in));
-      } else {
-        // pageable memory: one contiguous copy (a strided copy from pageable
-        // memory goes row by row through the runtime's staging)
-        P2Z_HIP_CHECK(hipMemcpyAsync(c->slot_hit[i], (const char*)hit + e0 * hit_ev, ne * hit_ev,
-                                     hipMemcpyHostToDevice, c->pipe_in));
+        // read, OMP:510-512); one row per record
+        P2Z_HIP_CHECK(hipMemcpy2DAsync(c->slot_hit[i], hit_rec, src_hit, stage_hit ? hit_used : hit_rec, hit_used,
+                                       (size_t)(n * nlayer), hipMemcpyHostToDevice, c->pipe_in));
+      } else if (nlayer > 0) {
+        P2Z_HIP_CHECK(hipMemcpyAsync(c->slot_hit[i], src_hit, n * hit_blk, hipMemcpyHostToDevice, c->pipe_in));
       }
       P2Z_HIP_CHECK(hipEventRecord(c->ev_in[i], c->pipe_in));
+      if (reuse && stage_dst) P2Z_TRY(drain(k - ns));
       hipStream_t s = c->pipe[i];
       P2Z_HIP_CHECK(hipStreamWaitEvent(s, c->ev_in[i], 0));
       if (reuse) P2Z_HIP_CHECK(hipStreamWaitEvent(s, c->ev_out[i], 0));
       P2Z_HIP_CHECK(p2z::launch_fused((const float*)c->slot_trk[i], (const float*)c->slot_hit[i],
-                                      (float*)c->slot_out[i], ne * nb, nlayer, width, math, c->cfg, s));
+                                      (float*)c->slot_out[i], n, nlayer, width, math, c->cfg, s));
       P2Z_HIP_CHECK(hipEventRecord(c->ev_done[i], s));
       P2Z_HIP_CHECK(hipStreamWaitEvent(c->pipe_out, c->ev_done[i], 0));
-      P2Z_HIP_CHECK(hipMemcpyAsync((char*)out + e0 * trk_ev, c->slot_out[i], ne * trk_ev,
-                                   hipMemcpyDeviceToHost, c->pipe_out));
+      P2Z_HIP_CHECK(hipMemcpyAsync(stage_dst ? (void*)c->stage_out[i] : (char*)out + b0 * trk_blk, c->slot_out[i],
+                                   n * trk_blk, hipMemcpyDeviceToHost, c->pipe_out));
       P2Z_HIP_CHECK(hipEventRecord(c->ev_out[i], c->pipe_out));
     }
+    if (stage_dst)
+      for (int64_t k = std::max<int64_t>(0, nchunks - ns); k < nchunks; ++k) P2Z_TRY(drain(k));
     return P2Z_OK;
   }();
   const hipError_t e = sync_pipeline(c);

@@ -3,9 +3,11 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <memory>
 #include <tuple>
 #include <vector>
 
+#include "p2z_copy.hpp"
 #include "p2z_internal.hpp"
 
 struct p2z_ctx {
@@ -22,6 +24,11 @@ struct p2z_ctx {
   // host-buffer pipeline staging, one slot per compute stream
   std::vector<void*> slot_trk, slot_hit, slot_out;
   size_t slot_trk_bytes = 0, slot_hit_bytes = 0;
+  // pinned staging of pageable host buffers, one slot per compute stream:
+  // tracks and the used hit words in, tracks out
+  std::vector<char*> stage_in, stage_out;
+  size_t stage_in_bytes = 0, stage_out_bytes = 0;
+  std::unique_ptr<p2z::CopyPool> copy;      // made by the first call that stages
   // device report scratch
   double* sum_part = nullptr;
   size_t sum_part_len = 0;
