@@ -58,8 +58,8 @@ typedef struct {
   int32_t tracks_per_wg; /* workgroup size in tracks: 64, 128, 192 or 256; 0 = 256 */
   int32_t nstreams;      /* staging slots of the host-buffer pipeline; 0 = 4      */
   int32_t hit_stage;     /* hit-staging depth: layers of hits in flight ahead of
-                            the one being computed, 1 or 2; 0 = per mode
-                            (2 for P2Z_MATH_FP64GAIN, 1 otherwise)          */
+                            the one being computed, 1 or 2; 0 = by mode and
+                            size of the pass                                */
   int32_t reserved;
 } p2z_opts;
 

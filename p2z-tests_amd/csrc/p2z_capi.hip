@@ -91,6 +91,7 @@ void free_pipeline_slots(p2z_ctx* c) {
 
 int apply_opts(p2z_ctx* c, const p2z_opts* o) {
   LaunchCfg cfg;
+  cfg.cus = c->cus;
   int ns = 4;
   if (o) {
     if (o->tracks_per_wg != 0) {
@@ -165,6 +166,9 @@ static int create_impl(p2z_ctx** out, int device, const p2z_opts* opts) {
   if (rc == P2Z_OK) rc = p2z::hip_status(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
   if (rc == P2Z_OK) rc = p2z::hip_status(hipEventCreate(&c->t0), "hipEventCreate");
   if (rc == P2Z_OK) rc = p2z::hip_status(hipEventCreate(&c->t1), "hipEventCreate");
+  if (rc == P2Z_OK)
+    rc = p2z::hip_status(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device),
+                         "hipDeviceGetAttribute");
   if (rc == P2Z_OK) rc = noalloc_scratch_init(device);
   if (rc == P2Z_OK) rc = apply_opts(c, opts);
   if (rc == P2Z_OK) rc = p2z::hip_status(hipMalloc((void**)&c->sum_done, p2z::kSumDoneBytes), "hipMalloc");
@@ -178,9 +182,6 @@ static int create_impl(p2z_ctx** out, int device, const p2z_opts* opts) {
     rc = p2z::hip_status(hipHostGetDevicePointer((void**)&c->sum_dev, c->sum_host, 0), "hipHostGetDevicePointer");
   }
   if (rc == P2Z_OK) rc = p2z::hip_status(hipMalloc((void**)&c->counter, p2z::kQueueBytes), "hipMalloc");
-  if (rc == P2Z_OK)
-    rc = p2z::hip_status(hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device),
-                         "hipDeviceGetAttribute");
   if (rc != P2Z_OK) return rc;
   *out = owner.release();
   return P2Z_OK;

@@ -19,14 +19,23 @@ inline bool valid_math(int m) { return m >= 0 && m <= 2; }
 struct LaunchCfg {
   int tracks_per_wg = 256;  // threads per workgroup, one track per thread
   int hit_stage = 0;        // layers of hits in flight ahead of the computed one (1 or 2);
-                            // 0: per arithmetic mode (default_hit_stage)
+                            // 0: by arithmetic mode and size (default_hit_stage)
+  int cus = 0;              // compute units of the device
 };
 
-// Hit-staging depth of the fused pass when none is set: FAST runs 5 waves per
-// SIMD at depth 1 (89 VGPRs) against 4 at depth 2 (100) and measures 1-3%
-// faster; the reference mode (100 / 112 VGPRs) runs at depth 1; the FP64-gain mode (126 / 138 VGPRs: 4 waves
-// against 3) within 1% either way, and keeps depth 2.
-inline int default_hit_stage(int math) { return math == 2 ? 2 : 1; }
+// Hit-staging depth of the fused pass when none is set.  FAST and FP64GAIN: 2
+// while every SIMD holds at most 4 of the pass's waves, which the registers
+// allow at depth 2 as well (103 / 136 VGPRs): with few waves a layer's step is
+// shorter than the latency of its hits.  20 layers, W = 32, depth 1 against 2:
+//   waves       300        1500       3000       4050       5100      15000
+//   FAST      16.0 14.7  20.6 19.7  28.0 27.4  35.6 35.5  43.2 43.9  121.5 122.9 us
+//   FP64GAIN  18.5 17.0  29.2 27.2  41.6 40.3  53.5 53.4  66.2 65.9  194.7 196.7
+// Beyond that 1 (91 / 120 VGPRs: one more wave per SIMD).  The reference
+// typing's step is longer than the latency: always 1 (300 waves 21.5 against
+// 21.9, 1500 31.1 against 32.2).
+inline int default_hit_stage(int math, int64_t ntracks, int cus) {
+  return math != 1 && (ntracks + 63) / 64 <= (int64_t)16 * cus ? 2 : 1;
+}
 
 // Fused driver pass: ntracks = nblocks*W tracks, all with nlayer layers.
 hipError_t launch_fused(const float* trk, const float* hit, float* out, int64_t nblocks,
