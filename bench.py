@@ -396,8 +396,8 @@ def section_ingest(ctx, trk, hit, nevts: int, nb: int, nl: int, W: int, math: st
     out on separate streams so that the transfers overlap each other and the
     compute.  Timed with pinned and with pageable host memory, beside the
     parts alone (one H2D of the whole inputs, one D2H of the output, the
-    compute).  From pinned memory the pipeline copies only the 6 of 9 words
-    of each hit record that the path reads."""
+    compute).  The pipeline copies only the 6 of 9 words of each hit
+    record that the path reads."""
     tl = nevts * nb * W * nl
     out = np.empty_like(trk)
     hit_used = hit.nbytes * 6 // 9
@@ -415,7 +415,7 @@ def section_ingest(ctx, trk, hit, nevts: int, nb: int, nl: int, W: int, math: st
         return float(np.median(ts)) * 1e3
 
     ms = wall(lambda: ctx.run_host(trk, hit, out, nevts, nb, nl, W, math))
-    res["pageable"] = {"ms": round(ms, 3), "tl_per_s": tl / (ms * 1e-3), "h2d_bytes": trk.nbytes + hit.nbytes}
+    res["pageable"] = {"ms": round(ms, 3), "tl_per_s": tl / (ms * 1e-3), "h2d_bytes": trk.nbytes + hit_used}
     pt, ph, po = ctx.pinned_copy(trk), ctx.pinned_copy(hit), ctx.pinned_empty(trk.size)
     ms = wall(lambda: ctx.run_host(pt, ph, po, nevts, nb, nl, W, math))
     res["pinned"] = {"ms": round(ms, 3), "tl_per_s": tl / (ms * 1e-3), "h2d_bytes": trk.nbytes + hit_used,

@@ -25,12 +25,12 @@ struct LaunchCfg {
 
 // Hit-staging depth of the fused pass when none is set.  FAST and FP64GAIN: 2
 // while every SIMD holds at most 4 of the pass's waves, which the registers
-// allow at depth 2 as well (103 / 136 VGPRs): with few waves a layer's step is
+// allow at depth 2 as well (100 / 136 VGPRs): with few waves a layer's step is
 // shorter than the latency of its hits.  20 layers, W = 32, depth 1 against 2:
 //   waves       300        1500       3000       4050       5100      15000
 //   FAST      16.0 14.7  20.6 19.7  28.0 27.4  35.6 35.5  43.2 43.9  121.5 122.9 us
 //   FP64GAIN  18.5 17.0  29.2 27.2  41.6 40.3  53.5 53.4  66.2 65.9  194.7 196.7
-// Beyond that 1 (91 / 120 VGPRs: one more wave per SIMD).  The reference
+// Beyond that 1 (89 / 120 VGPRs: one more wave per SIMD).  The reference
 // typing's step is longer than the latency: always 1 (300 waves 21.5 against
 // 21.9, 1500 31.1 against 32.2).
 inline int default_hit_stage(int math, int64_t ntracks, int cus) {
