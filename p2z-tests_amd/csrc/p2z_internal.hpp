@@ -25,14 +25,14 @@ struct LaunchCfg {
 
 // Hit-staging depth of the fused pass when none is set.  FAST and FP64GAIN: 2
 // while every SIMD holds at most 4 of the pass's waves, which the registers
-// allow at depth 2 as well (100 / 136 VGPRs): with few waves a layer's step is
+// allow at depth 2 as well (103 / 136 VGPRs): with few waves a layer's step is
 // shorter than the latency of its hits.  20 layers, W = 32, depth 1 against 2:
-//   waves       300        1500       3000       4050       5100      15000
-//   FAST      16.0 14.7  20.6 19.7  28.0 27.4  35.6 35.5  43.2 43.9  121.5 122.9 us
-//   FP64GAIN  18.5 17.0  29.2 27.2  41.6 40.3  53.5 53.4  66.2 65.9  194.7 196.7
-// Beyond that 1 (89 / 120 VGPRs: one more wave per SIMD).  The reference
-// typing's step is longer than the latency: always 1 (300 waves 21.5 against
-// 21.9, 1500 31.1 against 32.2).
+//   waves       750        1500       3000       4050       5100      15000
+//   FAST      14.3 13.2  18.4 17.9  28.8 28.5  37.9 37.3  44.8 44.7  126.5 126.3 us
+//   FP64GAIN  16.7 15.7  26.5 25.9  42.9 43.2  56.3 56.1  68.7 68.7  197.1 197.4
+// Beyond that 1 (93 / 122 VGPRs; FAST: one more wave per SIMD).  The reference
+// typing's step is longer than the latency: always 1 (1500 waves 30.4 against
+// 31.3, 15000 209.8 against 212.0).
 inline int default_hit_stage(int math, int64_t ntracks, int cus) {
   return math != 1 && (ntracks + 63) / 64 <= (int64_t)16 * cus ? 2 : 1;
 }
