@@ -103,7 +103,11 @@ __device__ inline void redo_ref(Track& t, const float* __restrict__ tb, const fl
 // layer in two had none in flight).  Near the end the last record is read
 // again instead (at most kDepth times per track), and the last layers follow
 // the loop.  20 layers, W = 32: 1500 waves 19.75 -> 17.65 us FAST; 15000 waves
-// 121.2 -> 119.7 FAST, 204.4 -> 200.9 REF, 198.4 -> 196.1 FP64 gain.
+// 121.2 -> 118.0 FAST, 204.4 -> 200.9 REF, 198.4 -> 196.1 FP64 gain.
+// At depth 1 the end has one code path for one layer left and one for two, so
+// nothing is read again (of the FAST figure 119.6 -> 118.0); with the FP64 gain
+// steps the second path would take 130 VGPRs, 3 waves per SIMD instead of 4
+// (192.3 -> 193.2 us), and the last record is read again.
 template <int W, int kMath, int kDepth>
 __device__ __forceinline__ bool run_layers(Track& t, const float* __restrict__ hb, int n) {
   static_assert(kDepth == 1 || kDepth == 2, "prefetch depth 1 or 2");
@@ -120,10 +124,18 @@ __device__ __forceinline__ bool run_layers(Track& t, const float* __restrict__ h
       b = at(lay + 2);
       layer_step<kMath, false>(t, a, g);
     }
-    if (lay < n) {
+    if constexpr (kMath == kFp64Gain) {
+      if (lay < n) {
+        a = at(lay + 1);
+        layer_step<kMath, false>(t, b, g);
+        if (lay + 1 < n) layer_step<kMath, false>(t, a, g);
+      }
+    } else if (lay + 1 < n) {
       a = at(lay + 1);
       layer_step<kMath, false>(t, b, g);
-      if (lay + 1 < n) layer_step<kMath, false>(t, a, g);
+      layer_step<kMath, false>(t, a, g);
+    } else if (lay < n) {
+      layer_step<kMath, false>(t, b, g);
     }
   } else {
     Hit c = at(2);
