@@ -160,40 +160,101 @@ __device__ __forceinline__ bool run_layers(Track& t, const float* __restrict__ h
   return marked<kMath>(t, g);
 }
 
-// Ragged form of run_layers: lane layer counts n <= nmax differ, the loop
-// runs to nmax (the same for every lane of the wave) with one layer step per
-// iteration, each lane's loads and steps masked by its own n.  The hits of the
-// next kDepth layers are in flight while a layer is computed; a single step
-// instance keeps the register count down where the steps are masked.
-template <int W, int kMath, int kDepth>
-__device__ __forceinline__ bool run_layers_lanes(Track& t, const float* __restrict__ hb, int n, int nmax) {
-  static_assert(kDepth == 1 || kDepth == 2, "prefetch depth 1 or 2");
-  if (nmax <= 0) return false;
-  auto at = [&](int lay) { return load_hit<W>(hb + (int64_t)lay * (kHitWords * W)); };
-  Carry<kMath> g;
-  Hit h0{}, h1{}, h2{};
-  if (0 < n) h0 = at(0);
-  if (1 < n) h1 = at(1);
-  if (kDepth >= 2 && 2 < n) h2 = at(2);
-  if (0 < n) layer_step<kMath, true>(t, h0, g);
-  for (int lay = 1; lay < nmax; ++lay) {
-    h0 = h1;
-    if constexpr (kDepth >= 2) {
-      h1 = h2;
-      if (lay + 2 < n) h2 = at(lay + 2);
-    } else if (lay + 1 < n) {
-      h1 = at(lay + 1);
-    }
-    if (lay < n) layer_step<kMath, false>(t, h0, g);
-  }
-  return marked<kMath>(t, g);
+// Maximum of v over each group of kLanes lanes, in every lane of the group
+// (every lane of the wave must be active).
+template <int kLanes>
+__device__ inline int group_max(int v) {
+#pragma unroll
+  for (int o = kLanes / 2; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
+  return v;
 }
 
-// Maximum of v over the 64 lanes of the wave (every lane must be active).
-__device__ inline int wave_max(int v) {
+__device__ inline int64_t lane_i64(int64_t v, int lane) {
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, lane);
+  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)((uint64_t)v >> 32), lane);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// Ragged form of run_layers: every lane has its own layer count n, the loop
+// runs to the wave's largest with each lane's steps masked by its own n (all
+// lanes of the wave must be active).  The loads are never masked, so that
+// their number is the same on every path and a wait is for the layer it needs
+// only: past its block's largest count a lane reads its last record again, and
+// the lanes of a block with no layers read a live block's.  A rolled loop whose
+// loads were masked and moved from buffer to buffer took, 2 events of 26
+// layers with the FP64 gain steps, 21.7 us (now 20.7), 20 events FAST 18.8
+// (17.9), 4 events REF 28.8 (27.9), 300 events REF 172.7 (170.0), 500 events
+// FAST 185.6 (185.5).  Two layers ahead: 187.4, 20.6.
+template <int W, int kMath, int kDepth>
+__device__ __forceinline__ bool run_layers_lanes(Track& t, const float* __restrict__ hit, int64_t at, int n) {
+  static_assert(kDepth == 1 || kDepth == 2, "prefetch depth 1 or 2");
+  int m = group_max<(W < 64 ? W : 64)>(n);  // the block's, at most 64 lanes of it
+  int most = m;
+  if constexpr (W < 64) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
-  return __builtin_amdgcn_readfirstlane(v);
+    for (int o = 32; o >= W; o >>= 1) most = max(most, __shfl_xor(most, o));
+  }
+  const int nmax = __builtin_amdgcn_readfirstlane(most);
+  if (nmax <= 0) return false;
+  if constexpr (W < 64) {
+    const int from = __builtin_ctzll(__ballot(m > 0));
+    const int64_t other = lane_i64(at, from);
+    const int other_m = __builtin_amdgcn_readlane(m, from);
+    at = m > 0 ? at : other;
+    m = m > 0 ? m : other_m;
+  }
+  const float* hb = hit + at;
+  int loaded = 0;
+  auto next = [&]() {
+    const Hit h = load_hit<W>(hb);
+    hb += ++loaded < m ? kHitWords * W : 0;
+    return h;
+  };
+  Carry<kMath> g;
+  Hit a = next(), b = next();
+  int lay = 1;
+  if constexpr (kDepth == 1) {
+    if (0 < n) layer_step<kMath, true>(t, a, g);
+    for (; lay + 2 < nmax; lay += 2) {  // b holds layer lay
+      a = next();
+      if (lay < n) layer_step<kMath, false>(t, b, g);
+      b = next();
+      if (lay + 1 < n) layer_step<kMath, false>(t, a, g);
+    }
+    if constexpr (kMath == kFp64Gain) {  // ends as in run_layers
+      if (lay < nmax) {
+        a = next();
+        if (lay < n) layer_step<kMath, false>(t, b, g);
+        if (lay + 1 < n) layer_step<kMath, false>(t, a, g);
+      }
+    } else if (lay + 1 < nmax) {
+      a = next();
+      if (lay < n) layer_step<kMath, false>(t, b, g);
+      if (lay + 1 < n) layer_step<kMath, false>(t, a, g);
+    } else if (lay < n) {
+      layer_step<kMath, false>(t, b, g);
+    }
+  } else {
+    Hit c = next();
+    if (0 < n) layer_step<kMath, true>(t, a, g);
+    for (; lay + 4 < nmax; lay += 3) {  // b holds layer lay, c layer lay + 1
+      a = next();
+      if (lay < n) layer_step<kMath, false>(t, b, g);
+      b = next();
+      if (lay + 1 < n) layer_step<kMath, false>(t, c, g);
+      c = next();
+      if (lay + 2 < n) layer_step<kMath, false>(t, a, g);
+    }
+    if (lay < nmax) {  // at most 4 layers
+      a = next();
+      if (lay < n) layer_step<kMath, false>(t, b, g);
+      b = next();
+      if (lay + 1 < n) layer_step<kMath, false>(t, c, g);
+      if (lay + 2 < n) layer_step<kMath, false>(t, a, g);
+      if (lay + 3 < n) layer_step<kMath, false>(t, b, g);
+    }
+  }
+  return marked<kMath>(t, g);
 }
 
 // ---------------------------------------------------------------------------
@@ -236,7 +297,7 @@ __device__ __forceinline__ void ragged_item(const float* __restrict__ trk, const
   const bool valid = di < nblocks;
   Track t{};
   int n = 0;
-  const float* hb = hit;
+  int64_t ho = 0;
   const float* tb = trk;
   BlockDesc d{};
   if (valid) {
@@ -246,11 +307,11 @@ __device__ __forceinline__ void ragged_item(const float* __restrict__ trk, const
     n = lane_nlay[d.trk_block * W + l];
     n = n < d.nlayer ? n : d.nlayer;
     n = n > 0 ? n : 0;
-    hb = hit + d.hit_block * (kHitWords * W) + l;
+    ho = d.hit_block * (kHitWords * W) + l;
   }
-  const bool redo = run_layers_lanes<W, kMath, kPrefetch>(t, hb, n, wave_max(n));
+  const bool redo = run_layers_lanes<W, kMath, kPrefetch>(t, hit, ho, n);
   if constexpr (kMath == kRef)
-    if (valid && redo) redo_ref<W>(t, tb, hb, n);
+    if (valid && redo) redo_ref<W>(t, tb, hit + ho, n);
   if (valid) store_track<W>(t, out + d.out_block * (kTrkWords * W) + l);
 }
 
@@ -440,7 +501,7 @@ __device__ __forceinline__ void serve_item(const ServeLaunch& a, uint64_t k, int
   const bool valid = di < ndesc;
   Track t{};
   int n = 0;
-  const float* hb = a.hit;
+  int64_t ho = 0;
   const float* tin = a.trk;
   if (valid) {
     tin = a.trk + tb * (kTrkWords * W) + l;
@@ -448,11 +509,11 @@ __device__ __forceinline__ void serve_item(const ServeLaunch& a, uint64_t k, int
     n = a.lanes[tb * W + l];
     n = n < nl ? n : nl;
     n = n > 0 ? n : 0;
-    hb = a.hit + hblk * (kHitWords * W) + l;
+    ho = hblk * (kHitWords * W) + l;
   }
-  const bool redo = run_layers_lanes<W, kMath, kPrefetch>(t, hb, n, wave_max(n));
+  const bool redo = run_layers_lanes<W, kMath, kPrefetch>(t, a.hit, ho, n);
   if constexpr (kMath == kRef)
-    if (valid && redo) redo_ref<W>(t, tin, hb, n);
+    if (valid && redo) redo_ref<W>(t, tin, a.hit + ho, n);
   if (valid) store_track_through<W>(t, a.out + ob * (kTrkWords * W) + l);
   wait_stores();
   if (lane == 0) {
