@@ -862,6 +862,7 @@ __global__ __launch_bounds__(kSumThreads) void k_summary(const float* __restrict
 #pragma unroll
     for (int e = 0; e < kSumRms; ++e) own[kSumMeans + 3 + e] = m2[e];
   }
+  __syncthreads();
   if (threadIdx.x < 64) {
     // one store instruction for the partials, written through to where every
     // XCD sees them, and complete before the workgroup is counted
@@ -912,6 +913,7 @@ __global__ __launch_bounds__(kSumThreads) void k_summary(const float* __restrict
 #pragma unroll
     for (int e = 0; e < kSumRms; ++e) own[kSumMeans + 3 + e] = (double)sqrtf((float)(m2[e] / ngood));
   }
+  __syncthreads();
   if (threadIdx.x < 64) {
     if (threadIdx.x < kSumVals) sys_store(&res->bits[threadIdx.x], __builtin_bit_cast(uint64_t, own[threadIdx.x]));
     wait_stores();
