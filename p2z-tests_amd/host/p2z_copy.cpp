@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <new>
 #include <system_error>
 
 namespace p2z {
@@ -39,10 +40,13 @@ void copy_row(char* dst, const char* src, size_t bytes) {
 
 CopyPool::CopyPool() {
   const int n = std::min(kMaxHelpers, processors() - 1);
+  // no exception leaves the constructor: it would destroy running threads
   try {
+    if (n > 0) helpers_.reserve(n);
     for (int i = 0; i < n; ++i) helpers_.emplace_back([this] { helper(); });
   } catch (const std::system_error&) {
     // no more threads to be had: the caller and those there are do the work
+  } catch (const std::bad_alloc&) {  // or no memory for one
   }
 }
 
