@@ -74,8 +74,25 @@ __device__ inline bool marked(const Track& t, const Carry<kMath>& g) {
     return false;
 }
 
+// Whether a wave leaves the reference typing's short layers after the first:
+// with one lane marked all are, since computing all of them again takes no
+// longer.
+template <int kMath>
+__device__ inline bool leaves(Carry<kMath>& g) {
+  if constexpr (kMath == kRef) {
+    if (any_lane(g.redo)) {
+      g.redo = true;
+      return true;
+    }
+  }
+  return false;
+}
+
 // The n layers of a marked track again, from its input state and in the full
-// form: the exception (an operand that overflows or is not finite).
+// form: the exception (an operand that overflows or is not finite).  128 waves,
+// 20 layers, W = 32: 20.9 us; 30 with an unused lane in every block (139 where
+// the short layers all came first and NaN took the calls of ref_rcp_any and
+// sincosf_large).
 template <int W>
 __device__ inline void redo_ref(Track& t, const float* __restrict__ tb, const float* __restrict__ hb, int n) {
   // the address hidden from common-subexpression elimination: otherwise the
@@ -118,6 +135,7 @@ __device__ __forceinline__ bool run_layers(Track& t, const float* __restrict__ h
   int lay = 1;
   if constexpr (kDepth == 1) {
     layer_step<kMath, true>(t, a, g);
+    if (leaves<kMath>(g)) n = 0;
     for (; lay + 2 < n; lay += 2) {  // b holds layer lay
       a = at(lay + 1);
       layer_step<kMath, false>(t, b, g);
@@ -140,6 +158,7 @@ __device__ __forceinline__ bool run_layers(Track& t, const float* __restrict__ h
   } else {
     Hit c = at(2);
     layer_step<kMath, true>(t, a, g);
+    if (leaves<kMath>(g)) n = 0;
     for (; lay + 4 < n; lay += 3) {  // b holds layer lay, c layer lay + 1
       a = at(lay + 2);
       layer_step<kMath, false>(t, b, g);
@@ -196,7 +215,7 @@ __device__ __forceinline__ bool run_layers_lanes(Track& t, const float* __restri
 #pragma unroll
     for (int o = 32; o >= W; o >>= 1) most = max(most, __shfl_xor(most, o));
   }
-  const int nmax = __builtin_amdgcn_readfirstlane(most);
+  int nmax = __builtin_amdgcn_readfirstlane(most);
   if (nmax <= 0) return false;
   if constexpr (W < 64) {
     const int from = __builtin_ctzll(__ballot(m > 0));
@@ -217,6 +236,7 @@ __device__ __forceinline__ bool run_layers_lanes(Track& t, const float* __restri
   int lay = 1;
   if constexpr (kDepth == 1) {
     if (0 < n) layer_step<kMath, true>(t, a, g);
+    if (leaves<kMath>(g)) n = nmax = 0;
     for (; lay + 2 < nmax; lay += 2) {  // b holds layer lay
       a = next();
       if (lay < n) layer_step<kMath, false>(t, b, g);
@@ -239,6 +259,7 @@ __device__ __forceinline__ bool run_layers_lanes(Track& t, const float* __restri
   } else {
     Hit c = next();
     if (0 < n) layer_step<kMath, true>(t, a, g);
+    if (leaves<kMath>(g)) n = nmax = 0;
     for (; lay + 4 < nmax; lay += 3) {  // b holds layer lay, c layer lay + 1
       a = next();
       if (lay < n) layer_step<kMath, false>(t, b, g);

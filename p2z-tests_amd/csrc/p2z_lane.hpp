@@ -54,6 +54,13 @@ struct Hit {
   float xx, xy, yy;  // covariance elements 0..2 (xz, yz, zz are never read)
 };
 
+// Whether a condition holds in any active lane: a test for rare cases that
+// leaves the common path of a wave without a divergent branch.  Three of them
+// per layer instead of four divergent regions: with one wave per SIMD, 2016
+// tracks x 17 layers FAST 11.8 -> 11.2 us, 53000 tracks of 8-26 layers FP64GAIN
+// 22.8 -> 21.7; full passes unchanged.
+__device__ inline bool any_lane(bool c) { return __builtin_expect(__builtin_amdgcn_ballot_w64(c) != 0, 0); }
+
 // ---------------------------------------------------------------------------
 // kRef: reference typing
 // ---------------------------------------------------------------------------
@@ -76,10 +83,12 @@ __device__ inline float fast_rcp(float x) {
 __device__ __noinline__ float ref_rcp_any(float x) { return (float)(1. / (double)x); }
 __device__ __noinline__ float ref_inv_det_any(double det) { return (float)(1. / det); }
 
-// (float)(1. / (double)x), the reference's float reciprocals.
+// (float)(1. / (double)x), the reference's float reciprocals.  NaN stays with
+// fast_rcp, which returns one: the lanes of a partly used block turn to NaN on
+// their first layer and would call on every other.
 __device__ inline float ref_rcp(float x) {
   const float a = __builtin_fabsf(x);
-  if (__builtin_expect(!(a > 0x1p-100f && a < 0x1p100f), 0)) return ref_rcp_any(x);
+  if (__builtin_expect(a <= 0x1p-100f || a >= 0x1p100f, 0)) return ref_rcp_any(x);
   return fast_rcp(x);
 }
 
@@ -114,11 +123,14 @@ struct RefCarry {
 // first term is, x - y only if x is).  That holds while the Jacobian is
 // finite and the products with the zeros are zeros: ok is cleared where
 // operands are outside ranges that bound every Jacobian entry below 2^127
-// (|ipt|, |1/ipt|, |1/cosT|, |dz| < 2^30) or z is a zero (the update adds a
-// zero of either sign to it); where the update meets a value that is not
+// (|ipt|, |1/ipt|, |1/cosT|, |dz| < 2^30) or z is -0 (the update adds a zero of
+// either sign to it; +0 stays); where the update meets a value that is not
 // finite, or an operand is NaN, a diagonal entry of P or a position ends up
 // not finite and stays so, which the caller sees at the end (ref_finite).
-// Such tracks are computed again with the full form.
+// Such tracks are computed again with the full form.  A wave with one after
+// its first layer, as the unused lanes of a block are, leaves the short form
+// there; one marked later computes its short layers first (looking for it in
+// the layer loop costs the passes without one 1%).
 // Bound: VALU issue, 671 instructions per layer before, about 460 now, with the
 // branch-free sin/cos and the reciprocals above.  100 events x 9600 tracks x
 // 20 layers: 0.260-0.266 -> 0.202 ms; 7 x 5008 x 26 at W = 16: 41 -> 27 us.
@@ -136,17 +148,16 @@ __device__ inline void propagate_ref(Track& t, float hz, const RefCarry& carry, 
   const float deltaZ = zout - p[2];
   const float ipt = p[3];
   float sinP, cosP, sinT, cosT;
-  // sincosf_glibc of both angles with one branch for its rare range (a NaN
-  // comes out as NaN of either)
+  // sincosf_glibc of both angles with one branch for its rare range
   glibc_sincosf::sincosf_below_120(p[4], &sinP, &cosP);
   glibc_sincosf::sincosf_below_120(p[5], &sinT, &cosT);
-  if (__builtin_expect(!(fmaxf(__builtin_fabsf(p[4]), __builtin_fabsf(p[5])) < 120.f), 0)) {
-    if (!(__builtin_fabsf(p[4]) < 120.f)) {
+  if (__builtin_expect(fmaxf(__builtin_fabsf(p[4]), __builtin_fabsf(p[5])) >= 120.f, 0)) {
+    if (__builtin_fabsf(p[4]) >= 120.f) {
       const glibc_sincosf::Poly v = glibc_sincosf::sincosf_large(p[4]);
       sinP = v.s;
       cosP = v.c;
     }
-    if (!(__builtin_fabsf(p[5]) < 120.f)) {
+    if (__builtin_fabsf(p[5]) >= 120.f) {
       const glibc_sincosf::Poly v = glibc_sincosf::sincosf_large(p[5]);
       sinT = v.s;
       cosT = v.c;
@@ -163,7 +174,7 @@ __device__ inline void propagate_ref(Track& t, float hz, const RefCarry& carry, 
     ok &= __builtin_fabsf(ipt) < 0x1p30f;
     ok &= __builtin_fabsf(pt) < 0x1p30f;
     ok &= __builtin_fabsf(icosT) < 0x1p30f;
-    ok &= zout != 0.f;
+    ok &= __builtin_bit_cast(uint32_t, zout) != 0x80000000u;
   }
   // The turning angle of one layer and cosP sina: below 0.75 in every lane of
   // the wave (then |cosP sina| < 0.69), as layers a few ten cm apart have it,
@@ -263,7 +274,7 @@ __device__ inline void update_ref(Track& t, const Hit& h, bool& ok) {
     ok &= m > 0x1p-119f && m < 0x1p119f;
   } else {
     const double m = __builtin_fabs(det);
-    if (__builtin_expect(!(m > 0x1p-120 && m < 0x1p120), 0))
+    if (__builtin_expect(m <= 0x1p-120 || m >= 0x1p120, 0))
       s = ref_inv_det_any(det);
     else
       s = ref_inv_det(det);
@@ -316,7 +327,7 @@ __device__ inline void step_ref_full(Track& t, const Hit& h, const RefCarry& c) 
 }
 
 // After a full step: whether the short form may follow (z row and column +0,
-// no other entry -0).
+// no other entry -0, positions and diagonal finite: x - x is +0).
 __device__ inline bool ref_z0_holds(const Track& t) {
   uint32_t z = 0;
   bool ok = true;
@@ -330,7 +341,8 @@ __device__ inline bool ref_z0_holds(const Track& t) {
       else
         ok &= w != 0x80000000u;
     }
-  return ok && z == 0;
+  const float sum = (t.p[0] + t.p[1]) + (t.P[S(0, 0)] + t.P[S(1, 1)]) + (t.P[S(3, 3)] + t.P[S(4, 4)] + t.P[S(5, 5)]);
+  return ok && (z | __builtin_bit_cast(uint32_t, sum - sum)) == 0;
 }
 
 // Positions and diagonal finite (those of a track that ever met a value that
@@ -379,7 +391,9 @@ __device__ __forceinline__ double sgpr_const(double v) {
 
 __device__ inline void sincos_accurate(float xf, float* sp, float* cp) {
   if (!(__builtin_fabsf(xf) < 0x1p20f)) {  // large, infinite or NaN
-    sincosf_glibc(xf, sp, cp);
+    const glibc_sincosf::Poly v = glibc_sincosf::sincosf_large(xf);
+    *sp = v.s;
+    *cp = v.c;
     return;
   }
   const double x = (double)xf;
@@ -436,13 +450,6 @@ __device__ inline void sincos_unit(float x, float* sp, float* cp, float* omcp) {
   *omcp = -(u * pc);
   *cp = __builtin_fmaf(u, pc, 1.0f);
 }
-
-// Whether a condition holds in any active lane: a test for rare cases that
-// leaves the common path of a wave without a divergent branch.  Three of them
-// per layer instead of four divergent regions: with one wave per SIMD, 2016
-// tracks x 17 layers FAST 11.8 -> 11.2 us, 53000 tracks of 8-26 layers FP64GAIN
-// 22.8 -> 21.7; full passes unchanged.
-__device__ inline bool any_lane(bool c) { return __builtin_expect(__builtin_amdgcn_ballot_w64(c) != 0, 0); }
 
 // Values used as they are rounded here: no multiplication above is fused into
 // an addition below.  The empty asm leaves them unchanged.

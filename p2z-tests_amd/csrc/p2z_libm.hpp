@@ -156,14 +156,14 @@ __host__ __device__ inline void sincosf_below_120(float y, float* sp, float* cp)
   *cp = __builtin_bit_cast(float, c ^ (((q << 30) + 0x40000000u) & 0x80000000u));
 }
 
-// Everything else: finite |y| >= 120 through Payne-Hanek, infinity and NaN.
+// Everything else: finite |y| >= 120 through Payne-Hanek, infinity.
 // Kept out of line: inline, its 64-bit products would add their registers to
 // every layer loop that calls sincosf_glibc, where real arguments never reach
 // it.
 __host__ __device__ __attribute__((noinline)) inline Poly sincosf_large(float y) {
 #pragma clang fp contract(off)
   const uint32_t bits = __builtin_bit_cast(uint32_t, y);
-  if (top12(bits) >= 0x7f8u) return Poly{y - y, y - y};  // inf or NaN
+  if (top12(bits) >= 0x7f8u) return Poly{y - y, y - y};  // inf (or NaN)
   const LargeReduction red = reduce_large(bits);
   const int sgn = red.n + (int)(bits >> 31);  // glibc's index of the sign table
   const Poly p = sincos_reduced(red.r);
@@ -177,8 +177,8 @@ __host__ __device__ __attribute__((noinline)) inline Poly sincosf_large(float y)
 // sin(y) and cos(y) with glibc's bits.
 __host__ __device__ inline void sincosf_glibc(float y, float* sp, float* cp) {
   using namespace glibc_sincosf;
-  sincosf_below_120(y, sp, cp);
-  if (!(__builtin_fabsf(y) < 120.0f)) {
+  sincosf_below_120(y, sp, cp);  // NaN comes out as NaN
+  if (__builtin_fabsf(y) >= 120.0f) {
     const Poly p = sincosf_large(y);
     *sp = p.s;
     *cp = p.c;
