@@ -1,9 +1,9 @@
-"""What a track that is outside the reference typing's short layer step from its
-first layer on costs its wave (p2z-tests_amd/csrc/p2z_lane.hpp): the full steps
-alone, not the short layers and then the full ones.  Every wave alone on its
-SIMD, so that the time of the pass is the time of its slowest wave; a full
-layer step is below 1.5 short ones (671 against 460 instructions), both
-together above 2."""
+"""What a track that is outside the reference typing's short layer step costs its
+wave (p2z-tests_amd/csrc/p2z_lane.hpp): where it is from the first layer on, the
+full steps alone; where it is later, the short steps and then the full ones.
+Every wave alone on its SIMD, so that the time of the pass is the time of its
+slowest wave; a full layer step is below 1.5 short ones (671 against 460
+instructions)."""
 from __future__ import annotations
 
 import numpy as np
@@ -30,7 +30,12 @@ def _layer_at_z_zero(trk, hit):
     hit[:, 2, 2] = 0.0
 
 
-@pytest.mark.parametrize("change,most", [(_unused_lane, 1.7), (_not_finite, 1.7), (_layer_at_z_zero, 1.2)])
+def _hit_z_missing(trk, hit):
+    hit[:, 2, 2, 7] = np.nan
+
+
+@pytest.mark.parametrize("change,most", [(_unused_lane, 1.7), (_not_finite, 1.7), (_layer_at_z_zero, 1.2),
+                                         (_hit_z_missing, 2.7)])
 def test_cost_of_a_wave_with_a_track_outside(ctx, change, most):
     trk, hit, _, nb = p2z.generate("ref", 1, NB * W, W, NL)
     t, h = trk.reshape(nb, 28, W).copy(), hit.reshape(nb, NL, 9, W).copy()
