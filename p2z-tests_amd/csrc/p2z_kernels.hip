@@ -644,7 +644,7 @@ __global__ __launch_bounds__(256) void k_propagate(const float* inErr, const flo
   t.q = inChg[o];
   const float hz = msP[b * hs + 2 * W + l];
   if constexpr (kMath == kRef) {
-    bool unused = true;
+    bool unused = false;
     propagate_ref<false>(t, hz, ref_carry(t), unused);
   } else
     propagate_fast<false, kMath == kFp64Gain>(t, hz);
@@ -678,7 +678,7 @@ __global__ __launch_bounds__(256) void k_update(float* trkErr, float* inPar, con
   h.xy = hitErr[ho + W];
   h.yy = hitErr[ho + 2 * W];
   if constexpr (kMath == kRef) {
-    bool unused = true;
+    bool unused = false;
     update_ref<false>(t, h, unused);
   } else if constexpr (kMath == kFast)
     update_fast<false>(t, h);

@@ -121,7 +121,7 @@ struct RefCarry {
 // a partial sum that is not -0, which leaves the sum's bits as they are, so it
 // is left out; what it leaves keeps both properties (a sum is -0 only if its
 // first term is, x - y only if x is).  That holds while the Jacobian is
-// finite and the products with the zeros are zeros: ok is cleared where
+// finite and the products with the zeros are zeros: out is set where
 // operands are outside ranges that bound every Jacobian entry below 2^127
 // (|ipt|, |1/ipt|, |1/cosT|, |dz| < 2^30) or z is -0 (the update adds a zero of
 // either sign to it; +0 stays); where the update meets a value that is not
@@ -139,7 +139,7 @@ struct RefCarry {
 // above 120 took 40 events of the wide-range workload from 139 us to 164; with
 // the library's large-argument path in the layer they take 124.
 template <bool kZ0>
-__device__ inline void propagate_ref(Track& t, float hz, const RefCarry& carry, bool& ok) {
+__device__ inline void propagate_ref(Track& t, float hz, const RefCarry& carry, bool& out) {
 #pragma clang fp contract(off)
   float* p = t.p;
   float* P = t.P;
@@ -170,11 +170,11 @@ __device__ inline void propagate_ref(Track& t, float hz, const RefCarry& carry, 
   const float icosTk = (float)((double)icosT * carry.rkd);
   const float alpha = deltaZ * sinT * ipt * icosTk;
   if constexpr (kZ0) {
-    ok &= __builtin_fabsf(deltaZ) < 0x1p30f;
-    ok &= __builtin_fabsf(ipt) < 0x1p30f;
-    ok &= __builtin_fabsf(pt) < 0x1p30f;
-    ok &= __builtin_fabsf(icosT) < 0x1p30f;
-    ok &= __builtin_bit_cast(uint32_t, zout) != 0x80000000u;
+    out |= !(__builtin_fabsf(deltaZ) < 0x1p30f);
+    out |= !(__builtin_fabsf(ipt) < 0x1p30f);
+    out |= !(__builtin_fabsf(pt) < 0x1p30f);
+    out |= !(__builtin_fabsf(icosT) < 0x1p30f);
+    out |= __builtin_bit_cast(uint32_t, zout) == 0x80000000u;
   }
   // The turning angle of one layer and cosP sina: below 0.75 in every lane of
   // the wave (then |cosP sina| < 0.69), as layers a few ten cm apart have it,
@@ -259,7 +259,7 @@ __device__ inline void propagate_ref(Track& t, float hz, const RefCarry& carry, 
 }
 
 template <bool kZ0>
-__device__ inline void update_ref(Track& t, const Hit& h, bool& ok) {
+__device__ inline void update_ref(Track& t, const Hit& h, bool& out) {
 #pragma clang fp contract(off)
   float* p = t.p;
   float* P = t.P;
@@ -271,7 +271,7 @@ __device__ inline void update_ref(Track& t, const Hit& h, bool& ok) {
   if constexpr (kZ0) {
     s = ref_inv_det(det);
     const float m = __builtin_fabsf(s);  // s in range implies det in ref_inv_det's
-    ok &= m > 0x1p-119f && m < 0x1p119f;
+    out |= !(m > 0x1p-119f && m < 0x1p119f);
   } else {
     const double m = __builtin_fabs(det);
     if (__builtin_expect(m <= 0x1p-120 || m >= 0x1p120, 0))
@@ -321,7 +321,7 @@ __device__ inline RefCarry ref_carry(const Track& t) {
 
 // One layer in the full form.
 __device__ inline void step_ref_full(Track& t, const Hit& h, const RefCarry& c) {
-  bool unused = true;
+  bool unused = false;
   propagate_ref<false>(t, h.z, c, unused);
   update_ref<false>(t, h, unused);
 }
@@ -1027,10 +1027,10 @@ __device__ inline void layer_step(Track& t, const Hit& h, Carry<kMath>& g) {
 #pragma unroll
       for (int i = 0; i < 6; ++i) t.P[S(i, 2)] = 0.f;
     } else {
-      bool ok = true;
-      propagate_ref<true>(t, h.z, g, ok);
-      update_ref<true>(t, h, ok);
-      g.redo |= !ok;
+      bool bad = false;
+      propagate_ref<true>(t, h.z, g, bad);
+      update_ref<true>(t, h, bad);
+      g.redo |= bad;
     }
   } else if constexpr (kMath == kFast) {
     if constexpr (kFirst) trig_init<false>(t, g);
