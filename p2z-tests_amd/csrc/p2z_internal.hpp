@@ -24,15 +24,17 @@ struct LaunchCfg {
 };
 
 // Hit-staging depth of the fused pass when none is set.  FAST and FP64GAIN: 2
-// while every SIMD holds at most 4 of the pass's waves, which the registers
-// allow at depth 2 as well (103 / 136 VGPRs): with few waves a layer's step is
-// shorter than the latency of its hits.  20 layers, W = 32, depth 1 against 2:
-//   waves       750        1500       3000       4050       5100      15000
-//   FAST      14.3 13.2  18.4 17.9  28.8 28.5  37.9 37.3  44.8 44.7  126.5 126.3 us
-//   FP64GAIN  16.7 15.7  26.5 25.9  42.9 43.2  56.3 56.1  68.7 68.7  197.1 197.4
-// Beyond that 1 (93 / 122 VGPRs; FAST: one more wave per SIMD).  The reference
-// typing's step is longer than the latency: always 1 (1500 waves 30.4 against
-// 31.3, 15000 209.8 against 212.0).
+// up to 16 waves per CU: with few waves a layer's step is shorter than the
+// latency of its hits.  At depth 2 FAST still holds 4 waves per SIMD (103
+// VGPRs; 5 at depth 1, 92), so that all 16 run at once; FP64GAIN holds 3 (136;
+// 4 at depth 1, 122), and between 12 and 16 waves per CU its last waves start
+// late at depth 2, which costs what the hits in flight gain.  20 layers,
+// W = 32, 256 CUs, us at depth 1 / 2 (runs differ by up to 1%):
+//   waves          750        1500       3072       3600       4096       15000
+//   FAST       14.2 13.4  17.8 17.5  27.5 26.1  31.9 31.8  34.7 34.4  118.0 119.7
+//   FP64GAIN   16.5 16.4  27.0 26.2  41.6 40.7  51.3 50.6  54.4 53.7  196.1 197.4
+// Beyond that 1.  The reference typing's step is longer than the latency:
+// always 1 (1500 waves 30.4 against 31.3, 15000 209.8 against 212.0).
 inline int default_hit_stage(int math, int64_t ntracks, int cus) {
   return math != 1 && (ntracks + 63) / 64 <= (int64_t)16 * cus ? 2 : 1;
 }
