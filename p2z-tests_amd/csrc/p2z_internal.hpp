@@ -29,10 +29,11 @@ struct LaunchCfg {
 // VGPRs; 5 at depth 1, 92), so that all 16 run at once; FP64GAIN holds 3 (136;
 // 4 at depth 1, 122), and between 12 and 16 waves per CU its last waves start
 // late at depth 2, which costs what the hits in flight gain.  20 layers,
-// W = 32, 256 CUs, us at depth 1 / 2 (runs differ by up to 1%):
+// W = 32, the same buffers every pass, 256 CUs, us at depth 1 and 2 (runs
+// differ by up to 1%):
 //   waves          750        1500       3072       3600       4096       15000
-//   FAST       14.2 13.4  17.8 17.5  27.5 26.1  31.9 31.8  34.7 34.4  118.0 119.7
-//   FP64GAIN   16.5 16.4  27.0 26.2  41.6 40.7  51.3 50.6  54.4 53.7  196.1 197.4
+//   FAST       14.2 13.4  17.8 17.5  27.5 26.1  31.9 31.8  34.7 34.4  110.8 112.9
+//   FP64GAIN   16.5 16.4  27.0 26.2  41.6 40.7  51.3 50.6  54.4 53.7  179.5 179.2
 // Beyond that 1.  The reference typing's step is longer than the latency:
 // always 1 (1500 waves 30.4 against 31.3, 15000 209.8 against 212.0).
 inline int default_hit_stage(int math, int64_t ntracks, int cus) {
