@@ -173,9 +173,11 @@ typedef struct {
   int32_t event;     /* owning event                                      */
 } p2z_block_desc;
 
-#define P2Z_RAGGED_PERSISTENT 1u /* one persistent launch draining a work queue
-                                    (descriptor order = processing order);
-                                    otherwise one wave per 64 track slots     */
+#define P2Z_RAGGED_PERSISTENT 1u /* may run as one persistent launch draining a
+                                    work queue (descriptor order = processing
+                                    order): does so where p2z_ragged_opts sets
+                                    its shape; otherwise one wave per 64 track
+                                    slots                                     */
 #define P2Z_RAGGED_GRAPH 2u      /* launch through a captured hipGraph, cached
                                     per argument set (either form); a context
                                     keeps up to 64 sets and empties its cache
@@ -272,10 +274,11 @@ int p2z_workload_load(const char* path, p2z_workload** out);
  * of budget_bytes in HBM: a request is admitted when its result blocks fit,
  * otherwise p2z_server_submit returns P2Z_EBUSY (retry after releasing
  * results) or P2Z_EINVAL (it can never fit).  p2z_server_pump launches every
- * admitted request not yet running as one batch on a free stream (one
- * persistent launch, descriptors longest-first), so requests arriving while
- * others run are admitted as slots and memory free up and their work
- * overlaps on the device; it also collects finished batches.  Results stay
+ * admitted request not yet running as one batch on a free stream (one launch,
+ * descriptors longest-first; on the work queue where waves_per_cu or
+ * items_per_claim is set), so requests arriving while others run are admitted
+ * as slots and memory free up and their work overlaps on the device; it also
+ * collects finished batches.  Results stay
  * in the arena until p2z_server_release.  Per-lane arithmetic does not depend
  * on the batch: a request's result is the same alone and in any mix.
  * With P2Z_SERVE_RESIDENT the requests are served by a device-resident loop

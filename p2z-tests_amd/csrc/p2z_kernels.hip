@@ -201,12 +201,17 @@ __device__ inline int64_t lane_i64(int64_t v, int lane) {
 // their number is the same on every path and a wait is for the layer it needs
 // only: past its block's largest count a lane reads its last record again, and
 // the lanes of a block with no layers read a live block's.  A rolled loop whose
-// loads were masked and moved from buffer to buffer took, 2 events of 26
-// layers with the FP64 gain steps, 21.7 us (now 20.7), 20 events FAST 18.8
+// loads were masked and moved from buffer to buffer took, 16 events (54062
+// tracks) with the FP64 gain steps, 21.7 us (now 20.7), 20 events FAST 18.8
 // (17.9), 4 events REF 28.8 (27.9), 300 events REF 172.7 (170.0), 500 events
 // FAST 185.6 (185.5).  Two layers ahead: 187.4, 20.6.
 // Two layers ahead with two layers left reading on would cost 2000 events FAST
 // 0.825 ms on the queue (now 0.820; the rolled loop 0.814).
+// On the queue and in the resident loop it takes registers that the rolled loop
+// did not (FAST one layer ahead 99 against 93 VGPRs): with more than 16 waves
+// per CU, FAST loses 1-5% (500 events 205.5 against 201 us, 200 events 86
+// against 82).  Every other shape is level or gains (64 threads, 8 waves per CU
+// 231 against 239), and the loop's median at 20000 events/s is 1.5-2 us less.
 template <int W, int kMath, int kDepth>
 __device__ __forceinline__ bool run_layers_lanes(Track& t, const float* __restrict__ hit, int64_t at, int n) {
   static_assert(kDepth == 1 || kDepth == 2, "prefetch depth 1 or 2");

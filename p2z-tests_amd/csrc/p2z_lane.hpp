@@ -67,8 +67,8 @@ __device__ inline bool any_lane(bool c) { return __builtin_expect(__builtin_amdg
 
 // 1/x to the nearest float: the hardware reciprocal (1 ulp) refined by one
 // Newton step with a fused multiply-add, for |x| in [2^-100, 2^100].  Equal to
-// (float)(1. / (double)x) on every float of that range (checked on the GPU
-// over all mantissas and exponents): 1/x of a 24-bit x is never closer than
+// (float)(1. / (double)x) on every float of that range (all of them compared
+// by tests/test_reciprocals.py): 1/x of a 24-bit x is never closer than
 // 2^-49 to the middle of two floats, so the double division the reference
 // writes does not round twice.  The 1-ulp estimate alone is biased low and
 // would shift all tracks of an event, which share nearly the same ipt and
@@ -96,8 +96,9 @@ __device__ inline float ref_rcp(float x) {
 // reciprocal (error below 2^-24, measured) refined by two Newton steps, so
 // that its last rounding sees 1/det within 2^-86.  The float differs from the
 // correctly rounded quotient's only if 1/det lies that close to a boundary of
-// the rounding to double next to the middle of two floats; an enumeration of
-// the 2^25 such boundaries finds no double det whose reciprocal does.
+// the rounding to double next to the middle of two floats; of the 2^25 such
+// boundaries the nearest to a double's reciprocal is 2^-78 away
+// (tests/test_reciprocals.py).
 __device__ inline float ref_inv_det(double det) {
   double y = __builtin_amdgcn_rcp(det);
   y = __builtin_fma(__builtin_fma(-det, y, 1.0), y, y);

@@ -1,5 +1,5 @@
 // Serving loop: admission by an HBM output arena, continuous batching of
-// events into persistent launches on several streams, per-event timestamps
+// events into launches on several streams, per-event timestamps
 // (declared in include/p2z.h).
 #include <hip/hip_runtime.h>
 

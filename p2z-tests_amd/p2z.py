@@ -655,8 +655,11 @@ class Context:
                    persistent: bool = True, graph: bool = False, tracks_per_wg: int = 0, prefetch: int = 0,
                    waves_per_cu: int = 0, items_per_claim: int = 0) -> None:
         """All blocks of a descriptor table (device buffer of BlockDesc) through
-        their layers: one persistent work-queue launch (optionally replayed from
-        a captured hipGraph), or one wave per 64 track slots."""
+        their layers in one launch (graph=True: replayed from a captured
+        hipGraph).  persistent=True with waves_per_cu or items_per_claim set: a
+        persistent grid of that shape on the work queue; with neither set the
+        library chooses, and takes one wave per 64 track slots, as
+        persistent=False does."""
         _need(blocks, nblocks * C.sizeof(BlockDesc), "block descriptors")
         flags = (RAGGED_PERSISTENT if persistent else 0) | (RAGGED_GRAPH if graph else 0)
         o = RaggedOpts(tracks_per_wg, prefetch, waves_per_cu, items_per_claim)
