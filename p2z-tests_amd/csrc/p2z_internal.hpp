@@ -35,7 +35,7 @@ struct LaunchCfg {
 //   FAST       14.2 13.4  17.8 17.5  27.5 26.1  31.9 31.8  34.7 34.4  110.8 112.9
 //   FP64GAIN   16.5 16.4  27.0 26.2  41.6 40.7  51.3 50.6  54.4 53.7  179.5 179.2
 // Beyond that 1.  The reference typing's step is longer than the latency:
-// always 1 (1500 waves 30.4 against 31.3, 15000 209.8 against 212.0).
+// always 1 (1500 waves 31.1 against 32.2, 15000 195.4 against 199.8).
 inline int default_hit_stage(int math, int64_t ntracks, int cus) {
   return math != 1 && (ntracks + 63) / 64 <= (int64_t)16 * cus ? 2 : 1;
 }
