@@ -175,7 +175,7 @@ __device__ inline void propagate_ref(Track& t, float hz, const RefCarry& carry, 
     out |= !(__builtin_fabsf(ipt) < 0x1p30f);
     out |= !(__builtin_fabsf(pt) < 0x1p30f);
     out |= !(__builtin_fabsf(icosT) < 0x1p30f);
-    out |= __builtin_bit_cast(uint32_t, zout) == 0x80000000u;
+    out |= __builtin_amdgcn_classf(zout, 0x20);  // -0
   }
   // The turning angle of one layer and cosP sina: below 0.75 in every lane of
   // the wave (then |cosP sina| < 0.69), as layers a few ten cm apart have it,
@@ -328,7 +328,8 @@ __device__ inline void step_ref_full(Track& t, const Hit& h, const RefCarry& c) 
 }
 
 // After a full step: whether the short form may follow (z row and column +0,
-// no other entry -0, positions and diagonal finite: x - x is +0).
+// no other entry -0), and the positions are finite: they are not where P or the
+// hit was not.
 __device__ inline bool ref_z0_holds(const Track& t) {
   uint32_t z = 0;
   bool ok = true;
@@ -342,8 +343,8 @@ __device__ inline bool ref_z0_holds(const Track& t) {
       else
         ok &= w != 0x80000000u;
     }
-  const float sum = (t.p[0] + t.p[1]) + (t.P[S(0, 0)] + t.P[S(1, 1)]) + (t.P[S(3, 3)] + t.P[S(4, 4)] + t.P[S(5, 5)]);
-  return ok && (z | __builtin_bit_cast(uint32_t, sum - sum)) == 0;
+  const bool finite = __builtin_isfinite(t.p[0]) && __builtin_isfinite(t.p[1]);
+  return ok && finite && z == 0;
 }
 
 // Positions and diagonal finite (those of a track that ever met a value that
